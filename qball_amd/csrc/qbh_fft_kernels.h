@@ -35,13 +35,7 @@ constexpr int ZLPW = 4;    // z-pass lines per wavefront (16 per group)
 
 // per precision: lines per wavefront in the y and x passes, y-pass plane block
 template <typename T> struct Cfg;
-// x-pass rows per wavefront and launch tuning (compile-time knobs)
-#ifndef QBH_XR64
-#define QBH_XR64 4
-#endif
-#ifndef QBH_XR32
-#define QBH_XR32 4
-#endif
+// launch tuning (compile-time knobs)
 // x pass: slots whose sphere lines are loaded ahead (register buffers of GPW elements
 // each).  Measured on MI355X at Si512: two slots ahead slowed the FP32 x pass from 4.26
 // to 4.60 ms per Hψ at three waves per SIMD (register spills) and to 5.57 ms at two; FP64
@@ -86,7 +80,6 @@ template <typename T> struct Cfg;
 #define QBH_YLB32 1
 #endif
 template <> struct Cfg<double> {
-  static constexpr int XR = QBH_XR64;  // x pass: rows per wavefront (64 B row segments)
   static constexpr int XPF = QBH_XPF64;  // x pass: slots of sphere lines in flight
   static constexpr int XWPE = QBH_XWPE64;  // x pass: minimum waves per SIMD asked of the compiler
   static constexpr int ZB = QBH_YZB64;  // y pass: z-planes per workgroup (column segments)
@@ -94,13 +87,28 @@ template <> struct Cfg<double> {
   static constexpr int LPW = ZB * LB / 4;
 };
 template <> struct Cfg<float> {
-  static constexpr int XR = QBH_XR32;
   static constexpr int XPF = QBH_XPF32;
   static constexpr int XWPE = QBH_XWPE32;
   static constexpr int ZB = QBH_YZB32;
   static constexpr int LB = QBH_YLB32;
   static constexpr int LPW = ZB * LB / 4;
 };
+
+// x pass: rows per wavefront for edge n = N1*N2.  A row gives the wavefront N2 stage-A and N1
+// stage-B tasks, one per lane, so it takes as many rows as keep both within its 64 lanes, and
+// of those the fewest that cover n rows with as many workgroups (whole last workgroups on
+// cubic grids): 4 rows at 140 = 14*10, 5 at 120 = 12*10, 6 at 72 = 9*8, 8 at 64 = 8*8.  The
+// pass is bound by vector-instruction issue, so idle lanes cost their full share.  Against 4
+// rows at every edge (x pass of one local Hψ, MI355X): 64^3 128 bands 111 -> 87 us (FP32 53 ->
+// 40), 72^3 128 bands 149 -> 103 (FP32 79 -> 67), 60^3 64 bands 56 -> 47, 144^3 unchanged.
+constexpr int x_rows(int n1, int n2) {
+  const int most = 64 / (n1 > n2 ? n1 : n2);
+  const int nb = (n1 * n2 + 4 * most - 1) / (4 * most);
+  return (n1 * n2 + 4 * nb - 1) / (4 * nb);
+}
+
+// x pass: line elements per thread of the short variant, for spheres up to half the edge
+constexpr int x_short(int n, int yb) { return (yb * (n / 2) + NTHR - 1) / NTHR; }
 
 template <typename T>
 __device__ __forceinline__ const cplx<T>* twtab(const GridDev& g, int axis);
@@ -582,7 +590,7 @@ __attribute__((amdgpu_waves_per_eu(Cfg<T>::XWPE)))
 k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
          const double* __restrict__ v, double* __restrict__ out, const double* __restrict__ dens,
          int cplx_density) {
-  constexpr int LPW = Cfg<T>::XR;
+  constexpr int LPW = x_rows(N1, N2);
   constexpr int YB = LPW * NWAVE;
   constexpr int n = N1 * N2;
   constexpr int TA = LPW * N2, TB = LPW * N1;
@@ -615,7 +623,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   // repeated products twiddle_row forms, computed once instead of per slot (measured at
   // 140 = 14*10: x pass 6.24 -> 6.01 ms per FP64 Hψ).  Not for the FP64 kernels with the
   // full line-element count, which have no registers to spare.
-  constexpr int GS = (YB * (n / 2 + 8) + NTHR - 1) / NTHR;
+  constexpr int GS = x_short(n, YB);
   constexpr bool TWB = QBH_XTWB && (sizeof(T) == 4 || GPW <= GS);
   cplx<T> twb[IB][TWB ? N2 - 1 : 1];
   if constexpr (TWB && OP == X_VMUL) {
@@ -644,15 +652,13 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   }
 
   // The workgroup moves the sphere lines of its YB rows together: element q = tid + NTHR*k
-  // is row dy = q % YB (= tid % YB, as YB divides NTHR) of line lx = q / YB, so one load
-  // instruction covers YB consecutive rows of NTHR/YB lines (YB*sizeof(cplx) contiguous
-  // bytes per line) instead of each wavefront's LPW rows.  GPW (a launch parameter) covers
+  // is row dy = q % YB of line lx = q / YB, so one load instruction covers YB consecutive
+  // rows of NTHR/YB lines (YB*sizeof(cplx) contiguous bytes per line) instead of each
+  // wavefront's LPW rows.  GPW (a launch parameter) covers
   // nlx*YB elements.  LDS offset (relative to the first row buffer) and T2 offset within a
   // slot are computed once, and the loads and LDS stores are unconditional: an element past
   // the lines loads element 0 of the slot and stores it to this thread's dump entry after
   // the row buffers; a row past np1 loads element 0 into its own (never stored) row.
-  static_assert(NTHR % YB == 0, "rows per workgroup must divide the workgroup size");
-  const bool rowok = ywg + (int)(threadIdx.x % YB) < np1;
   const long sstride = (long)np2 * nlx * np1;
   const int ngw = nlx * YB;
   cplx<T>* rows = tw + n;  // row buffers of all wavefronts, row dy at dy * LD
@@ -663,7 +669,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   for (int k = 0; k < GPW; ++k) {
     const int q = threadIdx.x + k * NTHR;
     const int dy = q % YB, lx = q / YB;
-    const bool in = q < ngw;
+    const bool in = q < ngw, rowok = ywg + dy < np1;
     lofs[k] = in ? dy * LD + PD::idx(g.line_x[lx]) : DUMP + (int)threadIdx.x;
     gofs[k] = (in && rowok) ? (z * nlx + lx) * np1 + ywg + dy : 0;
     if (in && rowok) gok |= 1u << k;
@@ -1134,8 +1140,8 @@ void launch_yfwd(hipStream_t st, const GridDev& g, const PipelineArgs& a) {
 template <typename T, int OP, int N1, int N2>
 void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw, const double* in,
                double* out, const double* dens, int cplx_density) {
-  constexpr int n = N1 * N2, YB = Cfg<T>::XR * NWAVE;
-  constexpr int GS = (YB * (n / 2 + 8) + NTHR - 1) / NTHR, GF = (YB * n + NTHR - 1) / NTHR;
+  constexpr int n = N1 * N2, YB = x_rows(N1, N2) * NWAVE;
+  constexpr int GS = x_short(n, YB), GF = (YB * n + NTHR - 1) / NTHR;
   const dim3 grid(g.np2 * ((g.np1 + YB - 1) / YB), (a.nslots + spw - 1) / spw);
   // twiddles, row buffers and one dump entry per thread
   const size_t lds =
@@ -1152,7 +1158,7 @@ void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
 template <typename T, int N1, int N2>
 constexpr EdgeOps make_edge() {
   return EdgeOps{N1 * N2,
-                 Cfg<T>::XR,
+                 x_rows(N1, N2),
                  launch_zbwd<T, N1, N2, 144>,
                  launch_ybwd<T, N1, N2, 144>,
                  launch_yfwd<T, N1, N2, 144>,
