@@ -155,17 +155,17 @@ template <int N1, int N2, int ON = QBH_LDS_PAD> struct Pad {
 };
 
 // Wavefront-local transform of `nrows` (<= RPW) LDS rows of length n = N1*N2 at
-// buf + r*ld (padded layout, Pad<N1,N2>), natural order in and out, direction DIR:
+// buf + r*ld (padded layout, Pad<N1,N2,PAD>), natural order in and out, direction DIR:
 //   stage A: task (r, j2): DFT_N1 over x[j2 + N2*j1], twiddle W_n^{DIR j2 k1}, in place
 //   stage B: task (r, k1): DFT_N2 over the contiguous block N2*k1 + j2 -> X[k1 + N1*k2],
 //            held in registers until every lane has read its block, then stored at the
 //            natural positions.
-template <int N1, int N2, int RPW, int DIR, typename T>
+template <int N1, int N2, int RPW, int DIR, int PAD = QBH_LDS_PAD, typename T>
 __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const cplx<T>* tw,
                                          int lane) {
   constexpr int TA = RPW * N2, TB = RPW * N1;
   constexpr int IA = (TA + 63) / 64, IB = (TB + 63) / 64;
-  constexpr int S = N2 + Pad<N1, N2>::P;  // padded stride of the N2-blocks
+  constexpr int S = N2 + Pad<N1, N2, PAD>::P;  // padded stride of the N2-blocks
 #pragma unroll
   for (int ia = 0; ia < IA; ++ia) {
     const int t = lane + 64 * ia;
@@ -202,7 +202,7 @@ __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const 
     if (t < TB && r < nrows) {
       cplx<T>* row = buf + r * ld;
 #pragma unroll
-      for (int k2 = 0; k2 < N2; ++k2) row[Pad<N1, N2>::idx(k1 + N1 * k2)] = b[ib][k2];
+      for (int k2 = 0; k2 < N2; ++k2) row[Pad<N1, N2, PAD>::idx(k1 + N1 * k2)] = b[ib][k2];
     }
   }
   wave_sync();

@@ -59,6 +59,7 @@ static constexpr EdgeOps stockham_edge() {
                  launch_zfwd<T, 0, 0, NMAX>,
                  nullptr,
                  nullptr,
+                 nullptr,
                  nullptr};
 }
 static const EdgeOps kStockham[2][2] = {
@@ -140,7 +141,9 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
              : OP == X_STORE ? r->xstore
              : OP == X_DENSITY ? r->xdensity
                                : nullptr;
-  const int yb = (reg ? r->xr : Cfg<T>::LPW) * NWAVE;  // rows per workgroup
+  constexpr bool LOAD = OP == X_LOAD || OP == X_LOAD_REAL;
+  // rows per workgroup
+  const int yb = (reg || (LOAD && r) ? r->xr : Cfg<T>::LPW) * NWAVE;
   const int spw = (OP == X_DENSITY) ? a.nslots
                   : b->tune.x_spw > 0 ? std::min(b->tune.x_spw, a.nslots)
                                       : x_slots_per_wg(g, a.nslots, yb);
@@ -148,6 +151,8 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
     TimedLaunch tl(ctx, name);
     if (reg)
       reg(ctx->stream, g, a, spw, in, out, dens, cplx_density);
+    else if (LOAD && r)
+      r->xload(ctx->stream, g, a, spw, in, OP == X_LOAD_REAL, scale);
     else
       launch_x<T, OP>(ctx->stream, g, a, spw, in, out, dens, scale, cplx_density);
   }

@@ -893,6 +893,81 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 }
 
 // ------------------------------------------------------------------------------------
+// x pass of the forward transform from a grid in memory (f complex, or REAL: scale * f + 0i):
+// each wavefront reads its rows (one contiguous stretch of the grid, all of a lane's loads in
+// flight together), transforms them with the two-factor register transform and the workgroup
+// stores the nlx sphere lines, YB consecutive rows of a line at a time.  Bound by HBM: it
+// reads the grid and writes T2.  With the LDS Stockham pass it replaces at these edges (198 us
+// of it) a backward and a forward transform of 65 orbitals at 72^3 took 343 us, now 208 us.
+template <typename T, bool REAL, int N1, int N2, int GPW>
+__global__ void __launch_bounds__(NTHR)
+k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
+         const double* __restrict__ f, double scale) {
+  constexpr int LPW = x_rows(N1, N2), YB = LPW * NWAVE, n = N1 * N2;
+  using PD = Pad<N1, N2, QBH_XLDS_PAD>;
+  constexpr int LD = PD::row(n);
+  constexpr int EPL = (LPW * n + 63) / 64;  // row elements per lane
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int np1 = g.np1, np2 = g.np2, nlx = g.nlx;
+  cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int nyb = (np1 + YB - 1) / YB;
+  const int z = blockIdx.x / nyb;
+  const int ywg = (blockIdx.x % nyb) * YB;
+  const int y0 = ywg + wave * LPW;
+  const int nyl = max(0, min(LPW, np1 - y0));
+  const int s0 = blockIdx.y * slots_per_wg;
+  const int s1 = min(nslots, s0 + slots_per_wg);
+  const cplx<T>* twg = twtab<T>(g, 0);
+  for (int i = threadIdx.x; i < n; i += NTHR) tw[i] = twg[i];
+  cplx<T>* rows = tw + n;
+  cplx<T>* buf = rows + wave * LPW * LD;
+  const long N = (long)n * np1 * np2;
+  const long grow0 = ((long)z * np1 + y0) * n;
+  const int nel = nyl * n;
+  const long sstride = (long)np2 * nlx * np1;
+  const int ngw = nlx * YB;
+  int lofs[GPW], gofs[GPW];
+#pragma unroll
+  for (int k = 0; k < GPW; ++k) {
+    const int q = threadIdx.x + k * NTHR;
+    const int dy = q % YB, lx = q / YB;
+    const bool ok = q < ngw && ywg + dy < np1;
+    lofs[k] = ok ? dy * LD + PD::idx(g.line_x[lx]) : 0;
+    gofs[k] = ok ? (z * nlx + lx) * np1 + ywg + dy : -1;
+  }
+  __syncthreads();
+  for (int s = s0; s < s1; ++s) {
+    if (nel > 0) {
+      // clamped, branch-free loads: past the rows a lane rereads their last element
+      cplx<T> v[EPL];
+#pragma unroll
+      for (int k = 0; k < EPL; ++k) {
+        const long e = (long)s * N + grow0 + min(lane + 64 * k, nel - 1);
+        if constexpr (REAL) {
+          v[k] = {T(scale * f[e]), T(0)};
+        } else {
+          v[k] = {T(f[2 * e]), T(f[2 * e + 1])};
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < EPL; ++k) {
+        const int e = lane + 64 * k;
+        if (e < nel) buf[(e / n) * LD + PD::idx(e % n)] = v[k];
+      }
+    }
+    wave_sync();
+    rows_fft<N1, N2, LPW, -1, QBH_XLDS_PAD>(buf, nyl, LD, tw, lane);
+    __syncthreads();
+    cplx<T>* dst = t2 + s * sstride;
+#pragma unroll
+    for (int k = 0; k < GPW; ++k)
+      if (gofs[k] >= 0) dst[gofs[k]] = rows[lofs[k]];
+    __syncthreads();
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // z pass, forward: T1 columns -> z transform (exp(-i)) -> x 1/N -> unpack -> output.
 // store 0: out[n][G] = ((out + add32) + kin[G]*psi[n][G]) + value;
 // store 1: out[n][G] = value;
@@ -1068,6 +1143,9 @@ struct EdgeOps {
                  const double* in, double* out, const double* dens, int cplx_density);
   void (*xdensity)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
                    const double* in, double* out, const double* dens, int cplx_density);
+  // register x pass of the forward transform, from a complex or (scaled) real grid
+  void (*xload)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
+                const double* f, bool real_input, double scale);
 };
 
 // register-transform edges compiled by unit `part` (qbh_fft_edges.hip)
@@ -1156,6 +1234,20 @@ void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
 }
 
 template <typename T, int N1, int N2>
+void launch_xload2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
+                   const double* f, bool real_input, double scale) {
+  constexpr int n = N1 * N2, YB = x_rows(N1, N2) * NWAVE;
+  constexpr int GF = (YB * n + NTHR - 1) / NTHR;
+  const dim3 grid(g.np2 * ((g.np1 + YB - 1) / YB), (a.nslots + spw - 1) / spw);
+  const size_t lds = sizeof(cplx<T>) * ((size_t)n + (size_t)YB * Pad<N1, N2, QBH_XLDS_PAD>::row(n));
+  auto* t2 = static_cast<cplx<T>*>(a.t2);
+  if (real_input)
+    k_xload2<T, true, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
+  else
+    k_xload2<T, false, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
+}
+
+template <typename T, int N1, int N2>
 constexpr EdgeOps make_edge() {
   return EdgeOps{N1 * N2,
                  x_rows(N1, N2),
@@ -1165,7 +1257,8 @@ constexpr EdgeOps make_edge() {
                  launch_zfwd<T, N1, N2, 144>,
                  launch_x2<T, X_VMUL, N1, N2>,
                  launch_x2<T, X_STORE, N1, N2>,
-                 launch_x2<T, X_DENSITY, N1, N2>};
+                 launch_x2<T, X_DENSITY, N1, N2>,
+                 launch_xload2<T, N1, N2>};
 }
 
 }  // namespace qbh

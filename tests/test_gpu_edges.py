@@ -70,3 +70,42 @@ def test_register_edges(gpu_ctx, grid, nb, real):
                    oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)) <= 1e-12
     ham.close()
     basis.close()
+
+
+@pytest.mark.parametrize("grid", [(18, 20, 30), (40, 64, 36), (60, 72, 42), (88, 90, 50),
+                                  (110, 24, 144), (140, 66, 28), (256, 20, 18), (162, 30, 22)])
+@pytest.mark.parametrize("flags,tol", [(0, 1e-12), (0x10, 2e-6)])
+def test_forward_from_grid(gpu_ctx, grid, flags, tol):
+    """forward (Γ pairs with a lone last band, and single bands) and forward_real at short,
+    long and Stockham x edges, row counts that leave the last workgroup part empty."""
+    import torch
+    from oracle import fft as offt
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=25.0, nbands=5, seed=23, generate_psi=False)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut), *grid)
+    r = sysm.rods
+    basis = Basis(gpu_ctx, True, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+    rng = np.random.default_rng(24)
+    g = rng.standard_normal((3, basis.N)) + 1j * rng.standard_normal((3, basis.N))
+    gd = torch.from_numpy(g.view(np.float64).ravel().copy()).cuda()
+    out = torch.zeros(2 * basis.ngw * 5, dtype=torch.float64, device="cuda")
+    shape = (maps.np2, maps.np1, maps.np0)
+    for nb, pair in ((5, True), (3, False)):
+        basis.forward(gd.data_ptr(), nb, pair, out.data_ptr(), basis.ngw, flags)
+        gpu_ctx.sync()
+        got = from_dev(out[:2 * basis.ngw * nb], basis.ngw, nb)
+        for s in range(3):
+            ref = offt.forward(maps, g[s].reshape(shape), pair=pair)
+            ref = ref if pair else (ref,)
+            for j, c in enumerate(ref):
+                if (2 if pair else 1) * s + j < nb:
+                    assert rel_err(got[:, (2 if pair else 1) * s + j], c) <= tol
+    rho = rng.standard_normal(basis.N)
+    rd = real_to_dev(rho)
+    basis.forward_real(rd.data_ptr(), 2.5, out.data_ptr(), flags)
+    gpu_ctx.sync()
+    ref = offt.forward(maps, (2.5 * rho).astype(np.complex128).reshape(shape))
+    assert rel_err(from_dev(out[:2 * basis.ngw], basis.ngw, 1)[:, 0], ref) <= tol
+    basis.close()
