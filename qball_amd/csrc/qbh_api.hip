@@ -572,11 +572,23 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
     const double f = prefac * occ[n];
     fac[n] = f > 0.0 ? f : 0.0;
   }
-  double* dfac = nullptr;
   const bool pair = b->g.real;
   const int nslots = pair ? (nst + 1) / 2 : nst;
-  if (hipMalloc(&dfac, (nst + 4 * (size_t)nslots) * sizeof(double)) != hipSuccess)
-    return fail(c, QBH_ERR_ALLOC, "density factor allocation failed");
+  const long N = (long)b->g.np0 * b->g.np1 * b->g.np2;
+  // band and slot factors, and the partial grids of the slot ranges (at most 256 MiB and the
+  // caller's workspace cap; without memory for them, one range)
+  const size_t nfac = ((nst + 4 * (size_t)nslots + 31) / 32) * 32;
+  const size_t chunk = std::max<size_t>(1, c->ws_cap / slot_bytes(b, prec));
+  int parts = density_parts(b, (int)std::min<size_t>(nslots, chunk), prec,
+                            std::min<size_t>(c->ws_cap, size_t(256) << 20));
+  double* dfac = nullptr;
+  if (parts > 1)
+    dfac = static_cast<double*>(aux_get(c, (nfac + (size_t)parts * N) * sizeof(double)));
+  if (!dfac) {
+    parts = 1;
+    dfac = static_cast<double*>(aux_get(c, nfac * sizeof(double)));
+  }
+  if (!dfac) return fail(c, QBH_ERR_ALLOC, "density factor allocation failed");
   hipMemcpyAsync(dfac, fac.data(), nst * sizeof(double), hipMemcpyHostToDevice, c->stream);
   double* slotf = dfac + nst;
   int r = for_chunks(c, b, nslots, prec, [&](PipelineArgs& a, int s0) {
@@ -585,6 +597,8 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
     a.nst = nst;
     a.band0 = pair ? 2 * s0 : s0;
     a.mode = pair ? SLOT_PAIR : SLOT_COMPLEX;
+    a.dens_parts = std::min(parts, a.nslots);
+    a.dens_part = dfac + nfac;
     k_dens_facs<<<(a.nslots + 255) / 256, 256, 0, c->stream>>>(a.nslots, a.band0, nst, pair ? 1 : 0,
                                                                dfac, psi_dev, ld,
                                                                slotf + 4 * (size_t)s0);
@@ -592,12 +606,10 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
     return pipeline_x_density(c, b, a, slotf + 4 * (size_t)s0, rho_dev);
   });
   hipStreamSynchronize(c->stream);
-  hipFree(dfac);
   if (r) return r;
   return dev_check(c, "density");
 }
 
-// ------------------------------------------------------------------------------------
 // ------------------------------------------------------------------------------------
 __global__ void k_zaxpy(long n, double ar, double ai, const double* __restrict__ x, long ldx,
                         double* __restrict__ y, long ldy, int ngw) {

@@ -38,21 +38,27 @@ TimedLaunch::~TimedLaunch() {
 
 thread_local bool t_capturing = false;
 
-void* ws_get(Ctx* ctx, size_t bytes) {
-  if (bytes <= ctx->ws_bytes) return ctx->ws;
+static void* grow_workspace(Ctx* ctx, void*& ws, size_t& have, size_t bytes) {
+  if (bytes <= have) return ws;
   if (t_capturing) return nullptr;  // no free / malloc / synchronisation under capture
-  if (ctx->ws) {
+  if (ws) {
     hipStreamSynchronize(ctx->stream);
-    hipFree(ctx->ws);
-    ctx->ws = nullptr;
-    ctx->ws_bytes = 0;
+    hipFree(ws);
+    ws = nullptr;
+    have = 0;
   }
-  if (hipMalloc(&ctx->ws, bytes) != hipSuccess) {
-    ctx->ws = nullptr;
+  if (hipMalloc(&ws, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    ws = nullptr;
     return nullptr;
   }
-  ctx->ws_bytes = bytes;
-  return ctx->ws;
+  have = bytes;
+  return ws;
+}
+
+void* ws_get(Ctx* ctx, size_t bytes) { return grow_workspace(ctx, ctx->ws, ctx->ws_bytes, bytes); }
+void* aux_get(Ctx* ctx, size_t bytes) {
+  return grow_workspace(ctx, ctx->aux, ctx->aux_bytes, bytes);
 }
 
 }  // namespace qbh
@@ -106,6 +112,7 @@ extern "C" int qbh_ctx_destroy(qbh_ctx ctx) {
   if (ctx->c.ev_fork) hipEventDestroy(ctx->c.ev_fork);
   if (ctx->c.ev_join) hipEventDestroy(ctx->c.ev_join);
   if (ctx->c.ws) hipFree(ctx->c.ws);
+  if (ctx->c.aux) hipFree(ctx->c.aux);
   if (ctx->c.own_stream) hipStreamDestroy(ctx->c.stream);
   delete ctx;
   return QBH_OK;

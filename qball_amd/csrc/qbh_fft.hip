@@ -144,7 +144,7 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
   constexpr bool LOAD = OP == X_LOAD || OP == X_LOAD_REAL;
   // rows per workgroup
   const int yb = (reg || (LOAD && r) ? r->xr : Cfg<T>::LPW) * NWAVE;
-  const int spw = (OP == X_DENSITY) ? a.nslots
+  const int spw = OP == X_DENSITY ? (a.nslots + a.dens_parts - 1) / a.dens_parts
                   : b->tune.x_spw > 0 ? std::min(b->tune.x_spw, a.nslots)
                                       : x_slots_per_wg(g, a.nslots, yb);
   {
@@ -181,12 +181,33 @@ int pipeline_x_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, 
              ? xpass_t<double, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load")
              : xpass_t<float, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load");
 }
+int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
+  const GridDev& g = b->g;
+  const EdgeOps* r = b->tune.x_reg ? register_ops(g.np0, prec) : nullptr;
+  const int yb = (r ? r->xr : prec == PREC_FP64 ? Cfg<double>::LPW : Cfg<float>::LPW) * NWAVE;
+  const long rows = (long)g.np2 * ((g.np1 + yb - 1) / yb);
+  const long N = (long)g.np0 * g.np1 * g.np2;
+  long p = std::min<long>((4096 + rows - 1) / rows, 16);
+  p = std::min<long>({p, nslots / 4, (long)(cap_bytes / (8 * (size_t)N))});
+  return (int)std::max<long>(p, 1);
+}
+
 int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* dens,
                        double* rho) {
   const int cd = a.mode == SLOT_COMPLEX ? 1 : 0;
-  return a.prec == PREC_FP64
-             ? xpass_t<double, X_DENSITY>(ctx, b, a, nullptr, rho, dens, 1.0, cd, "xpass_density")
-             : xpass_t<float, X_DENSITY>(ctx, b, a, nullptr, rho, dens, 1.0, cd, "xpass_density");
+  // slot ranges actually used (every one non-empty)
+  const int spw = (a.nslots + a.dens_parts - 1) / a.dens_parts;
+  const int parts = (a.nslots + spw - 1) / spw;
+  double* out = parts > 1 ? a.dens_part : rho;
+  const int r =
+      a.prec == PREC_FP64
+          ? xpass_t<double, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density")
+          : xpass_t<float, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density");
+  if (r || parts == 1) return r;
+  const long N = (long)b->g.np0 * b->g.np1 * b->g.np2;
+  TimedLaunch tl(ctx, "density_sum");
+  k_density_sum<4><<<(unsigned)((N + NTHR - 1) / NTHR), NTHR, 0, ctx->stream>>>(N, parts, out, rho);
+  return check_launch(ctx, "density_sum");
 }
 
 }  // namespace qbh

@@ -411,7 +411,8 @@ template <typename T, int OP, int NMAX>
 __global__ void __launch_bounds__(NTHR)
 k_xpass(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
         const double* __restrict__ v,      // VMUL: potential; LOAD*: input grid
-        double* __restrict__ out,          // STORE: complex grid; DENSITY: rho
+        double* __restrict__ out,          // STORE: complex grid; DENSITY: rho, or one
+                                           // partial grid per slot range (gridDim.y > 1)
         const double* __restrict__ dens,   // DENSITY: per slot (fac1, fac2, beta1, beta2)
         double scale, int cplx_density) {
   constexpr int LPW = Cfg<T>::LPW;
@@ -565,10 +566,11 @@ k_xpass(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
     wave_sync();
   }
   if (OP == X_DENSITY) {
+    double* o = out + blockIdx.y * N + grow0;
 #pragma unroll
     for (int k = 0; k < EPL; ++k) {
       const int e = lane + k * 64;
-      if (e < nel) out[grow0 + e] += acc[k];
+      if (e < nel) o[e] = gridDim.y > 1 ? acc[k] : o[e] + acc[k];
     }
   }
 }
@@ -880,13 +882,17 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
       if (s + d < s1) run_slot(s + d, pf[d]);
   }
   if (OP == X_DENSITY) {
+    double* o = out + (long)blockIdx.y * n * np1 * np2 + grow0;
 #pragma unroll
     for (int ib = 0; ib < IB; ++ib) {
       const int t = lane + 64 * ib;
       const int r = t / N1, k1 = t % N1;
       if (t < TB && r < nyl) {
 #pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) out[grow0 + r * n + k1 + N1 * k2] += acc[ib][k2];
+        for (int k2 = 0; k2 < N2; ++k2) {
+          double* e = o + r * n + k1 + N1 * k2;
+          *e = gridDim.y > 1 ? acc[ib][k2] : *e + acc[ib][k2];
+        }
       }
     }
   }
@@ -1123,6 +1129,26 @@ k_zpass_fwd(GridDev g, const cplx<T>* __restrict__ t1, const double* __restrict_
       }
     }
   }
+}
+
+// ------------------------------------------------------------------------------------
+// rho += sum of the nparts partial grids, in slot order (bound by HBM: nparts + 2 grids)
+template <int U>
+__global__ void __launch_bounds__(NTHR)
+k_density_sum(long N, int nparts, const double* __restrict__ part, double* __restrict__ rho) {
+  const long i = blockIdx.x * (long)NTHR + threadIdx.x;
+  if (i >= N) return;
+  double r = rho[i];
+  int p = 0;
+  for (; p + U <= nparts; p += U) {  // U partials in flight together
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = part[(p + u) * N + i];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r += v[u];
+  }
+  for (; p < nparts; ++p) r += part[p * N + i];
+  rho[i] = r;
 }
 
 // ------------------------------------------------------------------------------------

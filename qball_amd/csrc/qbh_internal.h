@@ -106,6 +106,9 @@ struct Ctx {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   size_t ws_cap = size_t(8) << 30;  // cap on pipeline workspace
+  // second workspace, for what a call needs beside the transform workspace
+  void* aux = nullptr;
+  size_t aux_bytes = 0;
   // autotuner results per problem shape (key -> knob values)
   std::map<std::string, std::vector<int>> tune_cache;
   // this device's allocation-free transform scratch (device address of the file-scope
@@ -128,6 +131,9 @@ struct TimedLaunch {
 };
 
 void* ws_get(Ctx* ctx, size_t bytes);
+// the context's second workspace, grown on demand like the transform workspace; null if it
+// cannot be allocated.  One call's use of it ends with the call.
+void* aux_get(Ctx* ctx, size_t bytes);
 
 // Set (per host thread) while the multi-cell Hψ graph is being captured: every workspace,
 // table and handle must then already exist, so the growth paths (ws_get, grow), the
@@ -151,6 +157,10 @@ struct PipelineArgs {
   void* t2;
   hipEvent_t wait_z = nullptr;  // the forward z pass (which writes the output) waits on it
   const float* add32 = nullptr; // FP32 term (2*ngw floats per band) the forward z pass adds
+  // density: the slots are cut into dens_parts ranges, each summed by its own workgroups into
+  // a partial grid of dens_part (unused when dens_parts is 1)
+  int dens_parts = 1;
+  double* dens_part = nullptr;
 };
 
 int pipeline_bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a);
@@ -165,6 +175,11 @@ int pipeline_x_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, 
 int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* facs,
                        double* rho);
 size_t slot_bytes(const Basis* b, int prec);
+// Slot ranges of the density x pass for chunks of nslots slots: each workgroup sums all slots
+// of its rows, so the rows alone give np2 * np1 / rows-per-workgroup workgroups (216 at 72^3,
+// 1260 at 140^3: 2.5 rounds of two per CU).  Ranges for about 4096 workgroups, at least 4
+// slots each, with at most cap_bytes of partial grids.
+int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes);
 // S (M x N, ld M) = alpha * A^T B - a0 b0^T over the real view with K rows (real != 0, the
 // Γ metric when alpha = 2) or A^H B (complex, K rows); K-split dgemm/zgemm (qbh_dense.hip)
 int band_product(Ctx* c, void* blas, bool real, int M, int N, long K, const double* A, long lda,

@@ -109,3 +109,35 @@ def test_forward_from_grid(gpu_ctx, grid, flags, tol):
     ref = offt.forward(maps, (2.5 * rho).astype(np.complex128).reshape(shape))
     assert rel_err(from_dev(out[:2 * basis.ngw], basis.ngw, 1)[:, 0], ref) <= tol
     basis.close()
+
+
+@pytest.mark.parametrize("real,nb", [(True, 15), (True, 16), (True, 45), (False, 9), (False, 23)])
+@pytest.mark.parametrize("grid", [(36, 40, 42), (22, 24, 18)])
+def test_density_slot_ranges(real, nb, grid):
+    """Density summed over slot ranges (counts that do not divide into them, lone last band,
+    empty bands), in one chunk and in chunks too small for ranges, added to what rho holds."""
+    import torch
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Context
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=25.0, nbands=nb, seed=25, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), *grid)
+    occ = np.where(np.arange(nb) % 5 == 3, 0.0, 1.0 + 0.1 * np.arange(nb))
+    ref = oh.compute_density(maps, sysm.psi, occ, 1.0, sysm.omega)
+    rng = np.random.default_rng(26)
+    r = sysm.rods
+    cd = to_dev(sysm.psi)
+    for cap in (8 << 30, 1 << 20):
+        ctx = Context(0, None)
+        ctx.set_workspace_cap(cap)
+        basis = Basis(ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+        start = rng.standard_normal(basis.N)
+        for flags, tol in ((0, 1e-12), (0x10, 2e-6)):
+            rho = real_to_dev(start)
+            torch.cuda.synchronize()
+            basis.density(cd.data_ptr(), basis.ngw, nb, occ, 1.0, sysm.omega, rho.data_ptr(), flags)
+            ctx.sync()
+            assert rel_err(rho.cpu().numpy() - start, ref) <= tol * 10  # start is ~10x ref
+        basis.close()
+        ctx.close()
