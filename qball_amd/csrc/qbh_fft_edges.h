@@ -5,20 +5,23 @@
 // make one LDS round trip per radix instead of three per transform pair: at 88^3 (108 Al
 // atoms, 195 bands, FP64, MI355X) the x pass took 1.37 ms and the y passes 0.30 / 0.26 ms per
 // Hψ on Stockham passes, and a two-cycle SCF 41.1 ms against 28.6 ms on the register ones.
+// FP32 takes the register transform only at the lengths marked E: at the D lengths (FP64
+// only) its twiddles, formed by repeated products, cost accuracy against the Stockham passes'
+// tabled ones (FP32 Hψ at 110^3: error 2.7e-8 against 2.2e-8 of the result).
 // Each QBH_EDGES_<p> is one compilation unit (qbh_fft_edges.hip with QBH_FFT_PART = p), the
 // lengths dealt so that the units take about the same time to compile.
 #pragma once
 
-#define QBH_EDGES_0(E) E(6, 3) E(9, 6) E(10, 9) E(14, 10)
-#define QBH_EDGES_1(E) E(5, 4) E(8, 7) E(12, 8) E(12, 12)
-#define QBH_EDGES_2(E) E(6, 4) E(10, 6) E(10, 10) E(15, 10)
-#define QBH_EDGES_3(E) E(7, 4) E(8, 8) E(12, 9) E(14, 11)
-#define QBH_EDGES_4(E) E(6, 5) E(11, 6) E(11, 10) E(16, 10)
-#define QBH_EDGES_5(E) E(8, 4) E(10, 7) E(14, 8) E(14, 12)
-#define QBH_EDGES_6(E) E(6, 6) E(9, 8) E(12, 10) E(16, 11)
-#define QBH_EDGES_7(E) E(8, 5) E(10, 8) E(14, 9) E(15, 12)
-#define QBH_EDGES_8(E) E(7, 6) E(12, 7) E(16, 8) E(16, 12)
-#define QBH_EDGES_9(E) E(11, 4) E(8, 6) E(11, 8) E(12, 11) E(15, 14)
-#define QBH_EDGES_10(E) E(10, 5) E(16, 14) E(16, 15)
-#define QBH_EDGES_11(E) E(16, 16)
+#define QBH_EDGES_0(E, D) D(6, 3) E(9, 6) E(10, 9) E(14, 10)
+#define QBH_EDGES_1(E, D) D(5, 4) D(8, 7) E(12, 8) E(12, 12)
+#define QBH_EDGES_2(E, D) D(6, 4) E(10, 6) E(10, 10) D(15, 10)
+#define QBH_EDGES_3(E, D) E(7, 4) E(8, 8) E(12, 9) D(14, 11)
+#define QBH_EDGES_4(E, D) D(6, 5) D(11, 6) D(11, 10) E(16, 10)
+#define QBH_EDGES_5(E, D) E(8, 4) D(10, 7) D(14, 8) E(14, 12)
+#define QBH_EDGES_6(E, D) E(6, 6) E(9, 8) E(12, 10) D(16, 11)
+#define QBH_EDGES_7(E, D) E(8, 5) E(10, 8) D(14, 9) E(15, 12)
+#define QBH_EDGES_8(E, D) D(7, 6) D(12, 7) E(16, 8) E(16, 12)
+#define QBH_EDGES_9(E, D) D(11, 4) E(8, 6) D(11, 8) D(12, 11) E(15, 14)
+#define QBH_EDGES_10(E, D) E(10, 5) E(16, 14) E(16, 15)
+#define QBH_EDGES_11(E, D) E(16, 16)
 #define QBH_EDGE_PARTS(P) P(0) P(1) P(2) P(3) P(4) P(5) P(6) P(7) P(8) P(9) P(10) P(11)
