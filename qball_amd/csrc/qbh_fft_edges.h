@@ -5,9 +5,9 @@
 // make one LDS round trip per radix instead of three per transform pair: at 88^3 (108 Al
 // atoms, 195 bands, FP64, MI355X) the x pass took 1.37 ms and the y passes 0.30 / 0.26 ms per
 // Hψ on Stockham passes, and a two-cycle SCF 41.1 ms against 28.6 ms on the register ones.
-// FP32 takes the register transform only at the lengths marked E: at the D lengths (FP64
-// only) its twiddles, formed by repeated products, cost accuracy against the Stockham passes'
-// tabled ones (FP32 Hψ at 110^3: error 2.7e-8 against 2.2e-8 of the result).
+// FP32 takes the register transform only at the E lengths: at the D lengths it keeps the
+// Stockham passes, whose tabled twiddles are more exact there than the repeated products of
+// the FP32 register transform (FP32 Hψ at 110^3: error 2.2e-8 against 2.7e-8 of the result).
 // Each QBH_EDGES_<p> is one compilation unit (qbh_fft_edges.hip with QBH_FFT_PART = p), the
 // lengths dealt so that the units take about the same time to compile.
 #pragma once

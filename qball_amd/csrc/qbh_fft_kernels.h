@@ -622,7 +622,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   T vr[IB][N2];
   double acc[IB][N2];
   // stage-B forward twiddles W_n^{-k1 m2}, m2 = 1..N2-1, of this lane's k1: the same
-  // repeated products twiddle_row forms, computed once instead of per slot (measured at
+  // factors twiddle_row forms, computed once instead of per slot (measured at
   // 140 = 14*10: x pass 6.24 -> 6.01 ms per FP64 Hψ).  Not for the FP64 kernels with the
   // full line-element count, which have no registers to spare.
   constexpr int GS = x_short(n, YB);
@@ -637,6 +637,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
       cplx<T> p = w;
 #pragma unroll
       for (int m = 1; m < N2; ++m) {
+        if constexpr (sizeof(T) == 8) p = {tw[k1 * m].x, -tw[k1 * m].y};
         twb[ib][m - 1] = p;
         if (m + 1 < N2) p = cmul(p, w);
       }
