@@ -97,14 +97,16 @@ template <> struct Cfg<float> {
 // x pass: rows per wavefront for edge n = N1*N2.  A row gives the wavefront N2 stage-A and N1
 // stage-B tasks, one per lane, so it takes as many rows as keep both within its 64 lanes, and
 // of those the fewest that cover n rows with as many workgroups (whole last workgroups on
-// cubic grids): 4 rows at 140 = 14*10, 5 at 120 = 12*10, 6 at 72 = 9*8, 8 at 64 = 8*8.  The
+// cubic grids): 4 rows at 140 = 14*10, 5 at 120 = 12*10, 6 at 72 = 9*8, 8 at 64 = 8*8.  Where
+// that saves less than an eighth of the workgroups (144 = 12*12: 8 against 9) it stays at 4,
+// whose 256-byte segments suit the memory better (500 Al atoms, whole FP64 Hψ: 5 rows 1 % slower).  The
 // pass is bound by vector-instruction issue, so idle lanes cost their full share.  Against 4
 // rows at every edge (x pass of one local Hψ, MI355X): 64^3 128 bands 111 -> 87 us (FP32 53 ->
 // 40), 72^3 128 bands 149 -> 103 (FP32 79 -> 67), 60^3 64 bands 56 -> 47, 144^3 unchanged.
 constexpr int x_rows(int n1, int n2) {
   const int most = 64 / (n1 > n2 ? n1 : n2);
-  const int nb = (n1 * n2 + 4 * most - 1) / (4 * most);
-  return (n1 * n2 + 4 * nb - 1) / (4 * nb);
+  const int nb = (n1 * n2 + 4 * most - 1) / (4 * most), nb4 = (n1 * n2 + 15) / 16;
+  return 8 * nb > 7 * nb4 ? 4 : (n1 * n2 + 4 * nb - 1) / (4 * nb);
 }
 
 // x pass: line elements per thread of the short variant, for spheres up to half the edge
