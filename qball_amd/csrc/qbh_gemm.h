@@ -7,7 +7,7 @@ namespace qbh {
 // Slices the reduction of an R x C output with reduction length Q is cut into (want > 0:
 // that many, else enough for ~2048 workgroups, each slice at least 512 long); the count
 // actually used (every slice non-empty).
-int mfma_slices(int R, int C, long Q, int want);
+int mfma_slices(bool fp32, int R, int C, long Q, int want);
 // Length of each slice for `slices` slices (a multiple of the 16-element stage).
 long mfma_slice_len(long Q, int slices);
 

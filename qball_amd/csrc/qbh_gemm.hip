@@ -10,8 +10,8 @@
 // c = k, q = p, X = F and Y = anl, which is c-contiguous (Y[q, c] at Y[c + q ldy]), so that
 // 16 lanes of one matrix-core result row store 16 consecutive coefficients of a band.
 //
-// Workgroup: 256 threads = 4 waves in a 2 x 2 arrangement, a 128 x 128 tile of C (each
-// wave 64 x 64 = 4 x 4 blocks of the 16 x 16 x 4 MFMA, 64 accumulators per lane), the
+// Workgroup: 256 threads = 4 waves in a 2 x 2 arrangement, a 128 x 128 tile of C (or 64 x 64
+// or 32 x 32 for small outputs, see tile_cost; each wave of the large tile 64 x 64 = 4 x 4 blocks of the 16 x 16 x 4 MFMA, 64 accumulators per lane), the
 // reduction in stages 16 deep double-buffered through LDS: each stage's global loads are
 // in flight while the previous stage's MFMAs run (64 per wave), one barrier per stage, two
 // workgroups per CU in FP64 and three in FP32.  The operands are read through buffer
@@ -42,7 +42,7 @@ namespace qbh {
 
 namespace {
 
-constexpr int kBR = 128, kBC = 128, kThreads = 256;
+constexpr int kThreads = 256;
 
 // stage depth (reduction elements per LDS stage) and waves per SIMD, per element type
 // (measured at the 512-atom Si shapes, F = anl^T psi / hpsi += anl F, buffer loads: FP64
@@ -82,7 +82,7 @@ template <> struct Mf<double> {
   typedef double2 v2;
   static constexpr int VN = 2;
   typedef double vn __attribute__((ext_vector_type(2)));
-  static constexpr int BQ = QBH_GEMM_BQ64, XS = BQ + 2, CS = kBC + (BQ == 32 ? 2 : 4);
+  static constexpr int BQ = QBH_GEMM_BQ64, XPAD = 2, CPAD = BQ == 32 ? 2 : 4;
   static constexpr int WPE = QBH_GEMM_WPE64;
   __device__ static acc op(double a, double b, acc c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -95,7 +95,7 @@ template <> struct Mf<float> {
   typedef float2 v2;
   static constexpr int VN = 4;
   typedef float vn __attribute__((ext_vector_type(4)));
-  static constexpr int BQ = QBH_GEMM_BQ32, XS = BQ + 4, CS = kBC + (BQ == 32 ? 2 : 4);
+  static constexpr int BQ = QBH_GEMM_BQ32, XPAD = 4, CPAD = BQ == 32 ? 2 : 4;
   static constexpr int WPE = QBH_GEMM_WPE32;
   __device__ static acc op(float a, float b, acc c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -190,21 +190,26 @@ __device__ inline __amdgpu_buffer_rsrc_t rsrc(const void* base, unsigned bytes) 
 // BUF (with XV and YV): the operands are read through buffer descriptors based at the
 // stage's first element, with per-lane offsets fixed for the whole reduction; the host
 // selects it when one stage of either operand spans less than kOutside bytes.
-template <typename T, bool YC, bool OUTC, bool XV, bool YV, bool BUF>
-__global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
+//
+// TB: 16 x 16 blocks per wave and direction (tile of 32 TB rows and columns); KS: BQ-deep
+// sub-stages per LDS stage.  Neither changes the order of the sum.
+template <typename T, bool YC, bool OUTC, bool XV, bool YV, bool BUF, int TB, int KS>
+__global__ void __launch_bounds__(kThreads, TB == 4 ? Mf<T>::WPE : KS > 1 ? 2 : 4) k_gemm(Args a) {
   using M = Mf<T>;
   using v2 = typename M::v2;
   using vn = typename M::vn;
   using acc_t = typename M::acc;
   constexpr int VN = M::VN;
-  constexpr int BQ = M::BQ;                    // stage depth
-  constexpr int QG = BQ / 4;                   // reduction indices per lane group and stage
-  constexpr int XS = M::XS, CS = M::CS;
-  constexpr int XTILE = kBR * XS;
-  constexpr int YTILE = YC ? BQ * CS : kBC * XS;
-  constexpr int NP = kBR * BQ / 2 / kThreads;  // element pairs per thread and operand
-  constexpr int PPR = BQ / 2;                  // pairs per q-contiguous row
-  constexpr int PPC = kBC / 2;                  // pairs per c-contiguous row (64)
+  constexpr int BT = 32 * TB;                  // tile rows and columns
+  constexpr int BQ = M::BQ;                    // sub-stage depth
+  constexpr int BS = BQ * KS;                  // LDS stage depth
+  constexpr int QG = BQ / 4;                   // reduction indices per lane group and sub-stage
+  constexpr int XS = BS + M::XPAD, CS = BT + M::CPAD;
+  constexpr int XTILE = BT * XS;
+  constexpr int YTILE = YC ? BS * CS : BT * XS;
+  constexpr int NP = BT * BS / 2 / kThreads;   // element pairs per thread and operand
+  constexpr int PPR = BS / 2;                  // pairs per q-contiguous row
+  constexpr int PPC = BT / 2;                  // pairs per c-contiguous row
   __shared__ __attribute__((aligned(16))) T lds[2 * (XTILE + YTILE)];
 
   const int nb8 = gridDim.x >> 3;
@@ -222,7 +227,7 @@ __global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
     tc = t % a.tiles_c;
     tr = t / a.tiles_c;
   }
-  const int r0 = tr * kBR, c0 = tc * kBC;
+  const int r0 = tr * BT, c0 = tc * BT;
   const long q0 = (long)s * a.qslice;
   const long q1 = min(a.Q, q0 + a.qslice);
 
@@ -259,10 +264,10 @@ __global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
         yin[it] = c0 + col < a.C;
       }
     }
-    const long rows = min(kBR, a.R - r0), cols = min(kBC, a.C - c0);
-    xext = (unsigned)(((rows - 1) * a.ldx + BQ) * (long)sizeof(T));
-    yext = YC ? (unsigned)(((BQ - 1) * a.ldy + cols) * (long)sizeof(T))
-              : (unsigned)(((cols - 1) * a.ldy + BQ) * (long)sizeof(T));
+    const long rows = min(BT, a.R - r0), cols = min(BT, a.C - c0);
+    xext = (unsigned)(((rows - 1) * a.ldx + BS) * (long)sizeof(T));
+    yext = YC ? (unsigned)(((BS - 1) * a.ldy + cols) * (long)sizeof(T))
+              : (unsigned)(((cols - 1) * a.ldy + BS) * (long)sizeof(T));
   }
 
   // staging: NP element pairs of X and of Y per thread and stage
@@ -320,41 +325,45 @@ __global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
     }
   };
 
-  acc_t acc[4][4];
+  acc_t acc[TB][TB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TB; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
-  auto compute = [&](int buf) {
-    const T* xl = lds + buf * (XTILE + YTILE);
-    const T* yl = xl + XTILE;
-    // VN MFMA steps per 16-byte fragment load
+  auto compute = [&](int buf, long left) {
 #pragma unroll
-    for (int jv = 0; jv < QG / VN; ++jv) {
-      vn xf[4], yf[4];
+    for (int ks = 0; ks < KS; ++ks) {
+      if (KS > 1 && ks * BQ >= left) break;
+      const T* xl = lds + buf * (XTILE + YTILE) + ks * BQ;
+      const T* yl = lds + buf * (XTILE + YTILE) + XTILE + ks * BQ * (YC ? CS : 1);
+      // VN MFMA steps per 16-byte fragment load
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
-        xf[bi] = *reinterpret_cast<const vn*>(xl + (wr * 64 + bi * 16 + l16) * XS + QG * lg +
-                                              VN * jv);
+      for (int jv = 0; jv < QG / VN; ++jv) {
+        vn xf[TB], yf[TB];
 #pragma unroll
-      for (int bj = 0; bj < 4; ++bj) {
-        if (YC) {
-          const T* p = yl + (QG * lg + VN * jv) * CS + wc * 64 + bj * 16 + l16;
+        for (int bi = 0; bi < TB; ++bi)
+          xf[bi] = *reinterpret_cast<const vn*>(xl + (wr * 16 * TB + bi * 16 + l16) * XS +
+                                                QG * lg + VN * jv);
 #pragma unroll
-          for (int e = 0; e < VN; ++e) yf[bj][e] = p[e * CS];
-        } else {
-          yf[bj] = *reinterpret_cast<const vn*>(yl + (wc * 64 + bj * 16 + l16) * XS + QG * lg +
-                                                VN * jv);
+        for (int bj = 0; bj < TB; ++bj) {
+          if (YC) {
+            const T* p = yl + (QG * lg + VN * jv) * CS + wc * 16 * TB + bj * 16 + l16;
+#pragma unroll
+            for (int e = 0; e < VN; ++e) yf[bj][e] = p[e * CS];
+          } else {
+            yf[bj] = *reinterpret_cast<const vn*>(yl + (wc * 16 * TB + bj * 16 + l16) * XS +
+                                                  QG * lg + VN * jv);
+          }
         }
+#pragma unroll
+        for (int e = 0; e < VN; ++e)
+#pragma unroll
+          for (int bi = 0; bi < TB; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < TB; ++bj)
+              acc[bi][bj] = M::op(xf[bi][e], yf[bj][e], acc[bi][bj]);
       }
-#pragma unroll
-      for (int e = 0; e < VN; ++e)
-#pragma unroll
-        for (int bi = 0; bi < 4; ++bi)
-#pragma unroll
-          for (int bj = 0; bj < 4; ++bj)
-            acc[bi][bj] = M::op(xf[bi][e], yf[bj][e], acc[bi][bj]);
     }
   };
 
@@ -365,10 +374,10 @@ __global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
   }
   __syncthreads();
   int buf = 0;
-  for (long qb = q0; qb < q1; qb += BQ) {
-    const bool more = qb + BQ < q1;
-    if (more) gload(xa, ya, qb + BQ);
-    compute(buf);
+  for (long qb = q0; qb < q1; qb += BS) {
+    const bool more = qb + BS < q1;
+    if (more) gload(xa, ya, qb + BS);
+    compute(buf, q1 - qb);
     if (more) lstore(xa, ya, buf ^ 1);
     __syncthreads();
     buf ^= 1;
@@ -377,11 +386,11 @@ __global__ void __launch_bounds__(kThreads, Mf<T>::WPE) k_gemm(Args a) {
   // epilogue: lane holds C[rb + M::row(lg, j)][cb + l16] of each block
   T* O = static_cast<T*>(a.O) + (long)s * a.ostride;
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
-    const int rb = r0 + wr * 64 + bi * 16;
+  for (int bi = 0; bi < TB; ++bi) {
+    const int rb = r0 + wr * 16 * TB + bi * 16;
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) {
-      const int c = c0 + wc * 64 + bj * 16 + l16;
+    for (int bj = 0; bj < TB; ++bj) {
+      const int c = c0 + wc * 16 * TB + bj * 16 + l16;
       if (c >= a.C) continue;
       const acc_t v = acc[bi][bj];
 #pragma unroll
@@ -413,8 +422,8 @@ __device__ inline T bload1(__amdgpu_buffer_rsrc_t r, unsigned off) {
   }
 }
 
-template <typename T, bool YC, bool OUTC>
-__global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
+template <typename T, bool YC, bool OUTC, int TB>
+__global__ void __launch_bounds__(kThreads, TB == 4 ? 2 : 4) k_gemm_direct(Args a) {
   using M = Mf<T>;
   using v2 = typename M::v2;
   using acc_t = typename M::acc;
@@ -423,8 +432,8 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
   constexpr int NP = QG / 2;
   constexpr unsigned SZ = sizeof(T);
   struct Stage {
-    T x[4][QG];
-    T y[4][QG];
+    T x[TB][QG];
+    T y[TB][QG];
   };
   const int nb8 = gridDim.x >> 3;
   const int bid = blockIdx.x;
@@ -441,7 +450,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
     tc = t % a.tiles_c;
     tr = t / a.tiles_c;
   }
-  const int r0 = tr * kBR, c0 = tc * kBC;
+  const int r0 = tr * 32 * TB, c0 = tc * 32 * TB;
   const long q0 = (long)s * a.qslice;
   const long q1 = min(a.Q, q0 + a.qslice);
   const T* __restrict__ X = static_cast<const T*>(a.X);
@@ -450,22 +459,22 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave >> 1, wc = wave & 1;
   const int l16 = lane & 15, lg = lane >> 4;
-  const int rw0 = r0 + wr * 64, cw0 = c0 + wc * 64;
+  const int rw0 = r0 + wr * 16 * TB, cw0 = c0 + wc * 16 * TB;
   const int rows = a.R - rw0, cols = a.C - cw0;
-  unsigned xo[4], yo[4];
-  bool xin[4], yin[4];
+  unsigned xo[TB], yo[TB];
+  bool xin[TB], yin[TB];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+  for (int b = 0; b < TB; ++b) {
     xo[b] = (unsigned)(((long)(b * 16 + l16) * a.ldx + QG * lg) * SZ);
     xin[b] = b * 16 + l16 < rows;
     yo[b] = YC ? (unsigned)(((long)(b * 16 + l16) + (long)QG * lg * a.ldy) * SZ)
                : (unsigned)(((long)(b * 16 + l16) * a.ldy + QG * lg) * SZ);
     yin[b] = b * 16 + l16 < cols;
   }
-  const unsigned xext = rows > 0 ? (unsigned)(((long)(min(64, rows) - 1) * a.ldx + BQ) * SZ) : 0u;
+  const unsigned xext = rows > 0 ? (unsigned)(((long)(min(16 * TB, rows) - 1) * a.ldx + BQ) * SZ) : 0u;
   const unsigned yext =
-      cols > 0 ? (YC ? (unsigned)(((long)(BQ - 1) * a.ldy + min(64, cols)) * SZ)
-                     : (unsigned)(((long)(min(64, cols) - 1) * a.ldy + BQ) * SZ))
+      cols > 0 ? (YC ? (unsigned)(((long)(BQ - 1) * a.ldy + min(16 * TB, cols)) * SZ)
+                     : (unsigned)(((long)(min(16 * TB, cols) - 1) * a.ldy + BQ) * SZ))
                : 0u;
 
   auto load = [&](Stage& st, long qb) {
@@ -474,7 +483,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
     const __amdgpu_buffer_rsrc_t ry =
         rsrc(YC ? Y + cw0 + qb * a.ldy : Y + qb + (long)cw0 * a.ldy, yext);
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < TB; ++b)
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
         const bool ok = xin[b] && QG * lg + 2 * p + 2 <= left;
@@ -483,7 +492,7 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
         st.x[b][2 * p + 1] = v.y;
       }
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < TB; ++b)
 #pragma unroll
       for (int p = 0; p < NP; ++p) {
         if (YC) {
@@ -500,18 +509,18 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
         }
       }
   };
-  acc_t acc[4][4];
+  acc_t acc[TB][TB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < TB; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
   auto mma = [&](const Stage& st) {
 #pragma unroll
     for (int j = 0; j < QG; ++j)
 #pragma unroll
-      for (int bi = 0; bi < 4; ++bi)
+      for (int bi = 0; bi < TB; ++bi)
 #pragma unroll
-        for (int bj = 0; bj < 4; ++bj) {
+        for (int bj = 0; bj < TB; ++bj) {
           acc[bi][bj] = M::op(st.x[bi][j], st.y[bj][j], acc[bi][bj]);
         }
   };
@@ -529,10 +538,10 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
   }
   T* O = static_cast<T*>(a.O) + (long)s * a.ostride;
 #pragma unroll
-  for (int bi = 0; bi < 4; ++bi) {
+  for (int bi = 0; bi < TB; ++bi) {
     const int rb = rw0 + bi * 16;
 #pragma unroll
-    for (int bj = 0; bj < 4; ++bj) {
+    for (int bj = 0; bj < TB; ++bj) {
       const int c = cw0 + bj * 16 + l16;
       if (c >= a.C) continue;
       const acc_t v = acc[bi][bj];
@@ -548,8 +557,50 @@ __global__ void __launch_bounds__(kThreads, 2) k_gemm_direct(Args a) {
   }
 }
 
-template <typename T, bool YC, bool OUTC>
-void launch(const Args& a, hipStream_t st) {
+// Tile choice.  A workgroup of tile tb takes us(tb) microseconds of its CU per reduction
+// element (measured on MI355X over projector shapes from 8 to 512 atoms: the 128 x 128 tile
+// has the most MFMAs per loaded element, the smaller ones waste less on edges and make enough
+// workgroups for small outputs), some 80 elements more for its start and end, and a fifth more
+// when it is alone on its CU.  The 256 CUs share the workgroups, and each slice's partial
+// output is written and read once.
+//   form                          us(4)   us(2)   us(1)
+//   FP64 F, through LDS           0.140   0.038   0.0115
+//   FP64 Hψ += βF, direct         0.122   0.045   0.022
+//   FP32, through LDS             0.070   0.0187  0.0056
+// Chosen and measured, against the 128 x 128 tile with its slices (us): F FP64 8 atoms 85 -> 4,
+// 64 atoms (256 x 128 x 18278) 95 -> 31, 108 atoms 135 -> 111, 216 atoms 567 -> 436; FP32 64
+// atoms 54 -> 23, 216 atoms 303 -> 240; Hψ += βF FP64 8 atoms 11 -> 4, FP32 64 atoms 28 -> 21.
+// 512 atoms keep the 128 x 128 tile (F 9.7 ms against 11.6 and 17 ms).
+struct Tiling {
+  int tb;      // tile = 32 tb rows and columns
+  int slices;  // reduction slices
+};
+
+enum Form { FORM_LDS64, FORM_DIRECT64, FORM_LDS32 };
+
+inline long tiles_of(int R, int C, int tb) {
+  const int t = 32 * tb;
+  return (long)((R + t - 1) / t) * ((C + t - 1) / t);
+}
+
+double tile_cost(Form f, int R, int C, long Q, int tb, long slices) {
+  static const double us[3][3] = {{0.140, 0.038, 0.0115}, {0.122, 0.045, 0.022},
+                                  {0.070, 0.0187, 0.0056}};
+  const long per_cu = (tiles_of(R, C, tb) * slices + 255) / 256;
+  const double u = us[f][tb == 4 ? 0 : tb == 2 ? 1 : 2] * (per_cu == 1 ? 1.2 : 1.0);
+  const double bytes = slices > 1 ? 2.0 * slices * R * (double)C * (f == FORM_LDS32 ? 4 : 8) : 0.0;
+  return per_cu * u * ((double)Q / slices + 80) + bytes / 4e6;
+}
+
+template <typename T, bool YC, bool OUTC, int TB>
+void launch(Args a, hipStream_t st, int slices) {
+  constexpr int BT = 32 * TB;
+  // the 32 x 32 tile, whose stages are bound by their latency, stages two sub-stages at a
+  // time (four, or two for the 64 x 64 tile, cost more in occupancy than they save)
+  constexpr int KS = TB == 1 ? 2 : 1;
+  a.tiles_r = (a.R + BT - 1) / BT;
+  a.tiles_c = (a.C + BT - 1) / BT;
+  a.nblocks = a.tiles_r * a.tiles_c * slices;
   const unsigned grid = (unsigned)((a.nblocks + 7) / 8 * 8);
   // pairs are aligned vectors, and a pair never straddles the end of the range, when the
   // leading dimension and the range along the pair (Q for q-contiguous reads, C for
@@ -557,36 +608,82 @@ void launch(const Args& a, hipStream_t st) {
   const bool xv = (a.ldx % 2) == 0 && (a.Q % 2) == 0;
   const bool yv = (a.ldy % 2) == 0 && ((YC ? (long)a.C : a.Q) % 2) == 0;
   // buffer addressing: a stage of each operand spans less than kOutside bytes
-  constexpr long BQ = Mf<T>::BQ;
-  const long xspan = ((kBR - 1) * a.ldx + BQ) * (long)sizeof(T);
-  const long yspan = (YC ? (BQ - 1) * a.ldy + kBC : (kBC - 1) * a.ldy + BQ) * (long)sizeof(T);
+  constexpr long BS = Mf<T>::BQ * KS;
+  const long xspan = ((BT - 1) * a.ldx + BS) * (long)sizeof(T);
+  const long yspan = (YC ? (BS - 1) * a.ldy + BT : (BT - 1) * a.ldy + BS) * (long)sizeof(T);
   const bool buf = QBH_GEMM_BUF && xv && yv && xspan < (long)kOutside && yspan < (long)kOutside;
   if constexpr (YC && sizeof(T) == 8) {
     if (buf && QBH_GEMM_DIRECT) {
-      k_gemm_direct<T, YC, OUTC><<<grid, kThreads, 0, st>>>(a);
+      k_gemm_direct<T, YC, OUTC, TB><<<grid, kThreads, 0, st>>>(a);
       return;
     }
   }
   if (buf)
-    k_gemm<T, YC, OUTC, true, true, true><<<grid, kThreads, 0, st>>>(a);
+    k_gemm<T, YC, OUTC, true, true, true, TB, KS><<<grid, kThreads, 0, st>>>(a);
   else if (xv && yv)
-    k_gemm<T, YC, OUTC, true, true, false><<<grid, kThreads, 0, st>>>(a);
+    k_gemm<T, YC, OUTC, true, true, false, TB, KS><<<grid, kThreads, 0, st>>>(a);
   else if (xv)
-    k_gemm<T, YC, OUTC, true, false, false><<<grid, kThreads, 0, st>>>(a);
+    k_gemm<T, YC, OUTC, true, false, false, TB, KS><<<grid, kThreads, 0, st>>>(a);
   else if (yv)
-    k_gemm<T, YC, OUTC, false, true, false><<<grid, kThreads, 0, st>>>(a);
+    k_gemm<T, YC, OUTC, false, true, false, TB, KS><<<grid, kThreads, 0, st>>>(a);
   else
-    k_gemm<T, YC, OUTC, false, false, false><<<grid, kThreads, 0, st>>>(a);
+    k_gemm<T, YC, OUTC, false, false, false, TB, KS><<<grid, kThreads, 0, st>>>(a);
+}
+
+template <bool YC, bool OUTC>
+void launch(const Args& a, hipStream_t st, bool fp32, int slices, int tb) {
+  if (fp32) {
+    if (tb == 4) launch<float, YC, OUTC, 4>(a, st, slices);
+    else if (tb == 2) launch<float, YC, OUTC, 2>(a, st, slices);
+    else launch<float, YC, OUTC, 1>(a, st, slices);
+  } else {
+    if (tb == 4) launch<double, YC, OUTC, 4>(a, st, slices);
+    else if (tb == 2) launch<double, YC, OUTC, 2>(a, st, slices);
+    else launch<double, YC, OUTC, 1>(a, st, slices);
+  }
+}
+
+// cheapest tile for a given slice count; the 128 x 128 tile unless another is an eighth cheaper
+int best_tile(Form f, int R, int C, long Q, long slices) {
+  int best = 4;
+  double cost = 0.875 * tile_cost(f, R, C, Q, 4, slices);
+  for (int tb : {2, 1}) {
+    const double c = tile_cost(f, R, C, Q, tb, slices);
+    if (c < cost) {
+      best = tb;
+      cost = c;
+    }
+  }
+  return best;
+}
+
+// tile and slices of the F product
+Tiling tiling(bool fp32, int R, int C, long Q) {
+  // about 2048 workgroups of the 128 x 128 tile, slices at least 512 long.  FP32 always cuts
+  // the sum here, so that its rounding does not depend on the tile.
+  const long tiles = tiles_of(R, C, 4);
+  const long s4 = std::max<long>(
+      1, std::min<long>({(2048 + tiles - 1) / tiles, 64, std::max<long>(1, Q / 512)}));
+  if (fp32) return {best_tile(FORM_LDS32, R, C, Q, s4), (int)s4};
+  Tiling best{4, (int)s4};
+  double cost = 0.875 * tile_cost(FORM_LDS64, R, C, Q, 4, s4);
+  for (int tb : {2, 1})
+    for (long s : {1, 2, 4, 8, 16, 24, 32, 48, 64}) {
+      if (Q / s < 64 && s > 1) break;
+      const double c = tile_cost(FORM_LDS64, R, C, Q, tb, s);
+      if (c < cost) {
+        best = {tb, (int)s};
+        cost = c;
+      }
+    }
+  return best;
 }
 
 }  // namespace
 
-int mfma_slices(int R, int C, long Q, int want) {
-  const long tiles = (long)((R + kBR - 1) / kBR) * ((C + kBC - 1) / kBC);
-  long s = want > 0 ? want : (2048 + tiles - 1) / tiles;
-  s = std::min<long>(s, 64);
-  s = std::min<long>(s, std::max<long>(1, Q / 512));  // at least 32 stages per slice
-  s = std::max<long>(1, s);
+int mfma_slices(bool fp32, int R, int C, long Q, int want) {
+  long s = want > 0 ? std::max<long>(1, std::min<long>({(long)want, 64, std::max<long>(1, Q / 512)}))
+                    : tiling(fp32, R, C, Q).slices;
   const long qs = ((Q + s - 1) / s + kBQ - 1) / kBQ * kBQ;
   return (int)((Q + qs - 1) / qs);
 }
@@ -611,15 +708,10 @@ int mfma_gemm_qq(hipStream_t st, bool fp32, int R, int C, long Q, const void* X,
   a.qslice = mfma_slice_len(Q, slices);
   if ((Q + a.qslice - 1) / a.qslice != slices) return -1;
   a.ostride = ostride;
-  a.tiles_r = (R + kBR - 1) / kBR;
-  a.tiles_c = (C + kBC - 1) / kBC;
-  a.nblocks = a.tiles_r * a.tiles_c * slices;
   a.r_fastest = 0;
   a.accumulate = 0;
-  if (fp32)
-    launch<float, false, false>(a, st);
-  else
-    launch<double, false, false>(a, st);
+  launch<false, false>(a, st, fp32, slices,
+                       best_tile(fp32 ? FORM_LDS32 : FORM_LDS64, R, C, Q, slices));
   return 0;
 }
 
@@ -638,15 +730,9 @@ int mfma_gemm_qc(hipStream_t st, bool fp32, int R, int C, long Q, const void* X,
   a.ldo = ldo;
   a.qslice = (Q + kBQ - 1) / kBQ * kBQ;
   a.ostride = 0;
-  a.tiles_r = (R + kBR - 1) / kBR;
-  a.tiles_c = (C + kBC - 1) / kBC;
-  a.nblocks = a.tiles_r * a.tiles_c;
   a.r_fastest = 1;
   a.accumulate = accumulate ? 1 : 0;
-  if (fp32)
-    launch<float, true, true>(a, st);
-  else
-    launch<double, true, true>(a, st);
+  launch<true, true>(a, st, fp32, 1, best_tile(fp32 ? FORM_LDS32 : FORM_DIRECT64, R, C, Q, 1));
   return 0;
 }
 

@@ -515,7 +515,7 @@ static int ensure_memory(qbh_td_s* t) {
   t->nrows = 0;
   for (qbh_species sp : h->sps) t->nrows += species_nproj(sp);
   const size_t rows_d = (size_t)t->nrows * t->ngw;
-  t->nsl = h->P > 0 ? mfma_slices(8 * h->P, t->order * t->nst, 2L * t->ngw, 16) : 1;
+  t->nsl = h->P > 0 ? mfma_slices(false, 8 * h->P, t->order * t->nst, 2L * t->ngw, 16) : 1;
   const size_t tabs[] = {rows_d, 3 * rows_d, 8 * (size_t)t->ngw * h->P,
                          8 * (size_t)h->P * t->nst * t->order,
                          8 * (size_t)h->P * t->nst * t->order,
