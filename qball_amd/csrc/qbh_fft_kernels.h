@@ -109,6 +109,23 @@ constexpr int x_rows(int n1, int n2) {
   return 8 * nb > 7 * nb4 ? 4 : (n1 * n2 + 4 * nb - 1) / (4 * nb);
 }
 
+// y pass: lines (z planes) per wavefront for edge n = N1*N2.  Filling the lanes as in the x
+// pass helps the short edges, whose passes are not yet bound by HBM, but only where the
+// workgroups' z blocks then cover n with fewer planes past its end (FP32: not more) than
+// blocks of 16, or exactly.  Backward / forward y pass of one local FP64 Hψ against 4 lines,
+// MI355X: 72^3 128 bands 68 / 66 -> 59 / 56 us, 64^3 128 bands 45 / 41 -> 41 / 36, 120^3 300 bands 543 /
+// 419 -> 484 / 391; without the rule 96^3 (5 lines: 100 planes) 342 -> 363 backward.
+template <typename T> constexpr int y_lines(int n1, int n2) {
+  const int n = n1 * n2, r = x_rows(n1, n2);
+  const int p4 = (n + 15) / 16 * 16, pr = (n + 4 * r - 1) / (4 * r) * 4 * r;
+  return pr < p4 || n % (4 * r) == 0 || (sizeof(T) == 4 && pr == p4) ? r : 4;
+}
+template <typename T, int N1, int N2> struct YCfg {
+  static constexpr int LPW = N1 > 0 ? y_lines<T>(N1 > 0 ? N1 : 1, N2 > 0 ? N2 : 1) : Cfg<T>::LPW;
+  static constexpr int LB = Cfg<T>::LB;
+  static constexpr int ZB = NWAVE * LPW / LB;
+};
+
 // x pass: line elements per thread of the short variant, for spheres up to half the edge
 constexpr int x_short(int n, int yb) { return (yb * (n / 2) + NTHR - 1) / NTHR; }
 
@@ -252,7 +269,7 @@ k_zpass_bwd(GridDev g, const double* __restrict__ psi, long ld, int nst, int ban
 template <typename T, int NMAX, int N1, int N2>
 __global__ void __launch_bounds__(NTHR)
 k_ypass_bwd(GridDev g, const cplx<T>* __restrict__ t1, cplx<T>* __restrict__ t2) {
-  constexpr int ZB = Cfg<T>::ZB, LB = Cfg<T>::LB, LPW = Cfg<T>::LPW;
+  constexpr int ZB = YCfg<T, N1, N2>::ZB, LB = YCfg<T, N1, N2>::LB, LPW = YCfg<T, N1, N2>::LPW;
   constexpr int EPL = Epl<LPW, NMAX>::v;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int np1 = g.np1, np2 = g.np2, nlx = g.nlx;
@@ -331,7 +348,7 @@ k_ypass_bwd(GridDev g, const cplx<T>* __restrict__ t1, cplx<T>* __restrict__ t2)
 template <typename T, int NMAX, int N1, int N2>
 __global__ void __launch_bounds__(NTHR)
 k_ypass_fwd(GridDev g, const cplx<T>* __restrict__ t2, cplx<T>* __restrict__ t1) {
-  constexpr int ZB = Cfg<T>::ZB, LB = Cfg<T>::LB, LPW = Cfg<T>::LPW;
+  constexpr int ZB = YCfg<T, N1, N2>::ZB, LB = YCfg<T, N1, N2>::LB, LPW = YCfg<T, N1, N2>::LPW;
   constexpr int EPL = Epl<LPW, NMAX>::v;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int np1 = g.np1, np2 = g.np2, nlx = g.nlx;
@@ -1222,13 +1239,13 @@ void launch_zfwd(hipStream_t st, const GridDev& g, const PipelineArgs& a, double
 template <typename T, int N1, int N2>
 size_t lds_y(const GridDev& g) {
   return sizeof(cplx<T>) *
-             ((size_t)g.np1 + (size_t)Cfg<T>::ZB * Cfg<T>::LB * Pad<N1, N2>::row(g.np1)) +
-         sizeof(int) * (size_t)Cfg<T>::LB * g.np1;
+             ((size_t)g.np1 + (size_t)NWAVE * YCfg<T, N1, N2>::LPW * Pad<N1, N2>::row(g.np1)) +
+         sizeof(int) * (size_t)YCfg<T, N1, N2>::LB * g.np1;
 }
 
 template <typename T, int N1, int N2, int NMAX>
 void launch_ybwd(hipStream_t st, const GridDev& g, const PipelineArgs& a) {
-  constexpr int ZB = Cfg<T>::ZB, LB = Cfg<T>::LB;
+  constexpr int ZB = YCfg<T, N1, N2>::ZB, LB = YCfg<T, N1, N2>::LB;
   const dim3 grid(((g.np2 + ZB - 1) / ZB) * ((g.nlx + LB - 1) / LB), a.nslots);
   k_ypass_bwd<T, NMAX, N1, N2><<<grid, NTHR, lds_y<T, N1, N2>(g), st>>>(
       g, static_cast<const cplx<T>*>(a.t1), static_cast<cplx<T>*>(a.t2));
@@ -1236,7 +1253,7 @@ void launch_ybwd(hipStream_t st, const GridDev& g, const PipelineArgs& a) {
 
 template <typename T, int N1, int N2, int NMAX>
 void launch_yfwd(hipStream_t st, const GridDev& g, const PipelineArgs& a) {
-  constexpr int ZB = Cfg<T>::ZB, LB = Cfg<T>::LB;
+  constexpr int ZB = YCfg<T, N1, N2>::ZB, LB = YCfg<T, N1, N2>::LB;
   const dim3 grid(((g.np2 + ZB - 1) / ZB) * ((g.nlx + LB - 1) / LB), a.nslots);
   k_ypass_fwd<T, NMAX, N1, N2><<<grid, NTHR, lds_y<T, N1, N2>(g), st>>>(
       g, static_cast<const cplx<T>*>(a.t2), static_cast<cplx<T>*>(a.t1));
