@@ -60,6 +60,7 @@ static constexpr EdgeOps stockham_edge() {
                  nullptr,
                  nullptr,
                  nullptr,
+                 nullptr,
                  nullptr};
 }
 static const EdgeOps kStockham[2][2] = {
@@ -206,8 +207,66 @@ int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* 
   if (r || parts == 1) return r;
   const long N = (long)b->g.np0 * b->g.np1 * b->g.np2;
   TimedLaunch tl(ctx, "density_sum");
-  k_density_sum<4><<<(unsigned)((N + NTHR - 1) / NTHR), NTHR, 0, ctx->stream>>>(N, parts, out, rho);
+  k_density_sum<4><<<(unsigned)((N + NTHR - 1) / NTHR), NTHR, 0, ctx->stream>>>(N, parts, 1.0, out,
+                                                                               rho);
   return check_launch(ctx, "density_sum");
+}
+
+bool cross_edge(const Basis* b) {
+  const EdgeOps* r = b->tune.x_reg ? register_ops(b->g.np0, PREC_FP64) : nullptr;
+  return r && r->xcross;
+}
+
+int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* const* bs,
+                   long ldb, int nbands, int nb, const double* w, double scale, double* out) {
+  const GridDev& g = b->g;
+  const EdgeOps* r = register_ops(g.np0, PREC_FP64);
+  const size_t c = sizeof(cplx<double>);
+  const size_t t1 = c * g.ncol * g.np2, t2 = c * g.np2 * g.nlx * g.np1;
+  const size_t per = t1 + (nb + 1) * t2;
+  const long N = (long)g.np0 * g.np1 * g.np2;
+  const int S = (int)std::min<size_t>({std::max<size_t>(1, ctx->ws_cap / per), (size_t)nbands, 65535});
+  char* ws = static_cast<char*>(ws_get(ctx, S * per));
+  // partial grids per slot range: one range at least, more as for the density
+  const size_t cap = std::min<size_t>(ctx->ws_cap, size_t(256) << 20) / nb;
+  int parts = density_parts(b, S, PREC_FP64, cap);
+  double* part = static_cast<double*>(aux_get(ctx, sizeof(double) * parts * nb * N));
+  if (!part && parts > 1)
+    part = static_cast<double*>(aux_get(ctx, sizeof(double) * (parts = 1) * nb * N));
+  if (!ws || !part) {
+    ctx->last_error = "transform workspace allocation failed";
+    return -2;
+  }
+  CrossFields f{};
+  for (int d = 0; d <= nb; ++d)
+    f.t2[d] = reinterpret_cast<cplx<double>*>(ws + S * (t1 + d * t2));
+  for (int n0 = 0; n0 < nbands; n0 += S) {
+    PipelineArgs p{};
+    p.nslots = std::min(S, nbands - n0);
+    p.nst = nbands;
+    p.band0 = n0;
+    p.mode = g.real ? SLOT_SINGLE_REAL : SLOT_COMPLEX;
+    p.prec = PREC_FP64;
+    p.t1 = ws;
+    for (int d = 0; d <= nb; ++d) {
+      p.psi = d ? bs[d - 1] : a;
+      p.ld = d ? ldb : lda;
+      p.t2 = const_cast<cplx<double>*>(f.t2[d]);
+      if (int e = pipeline_bwd_yz(ctx, b, p)) return e;
+    }
+    const int pn = std::min(parts, p.nslots);
+    const int spw = (p.nslots + pn - 1) / pn, used = (p.nslots + spw - 1) / spw;
+    {
+      TimedLaunch tl(ctx, "xpass_cross");
+      r->xcross(ctx->stream, g, f, p.nslots, spw, nb, w ? w + n0 : nullptr, part);
+    }
+    if (int e = check_launch(ctx, "xpass_cross")) return e;
+    TimedLaunch tl(ctx, "density_sum");
+    k_density_sum<4><<<(unsigned)((nb * N + NTHR - 1) / NTHR), NTHR, 0, ctx->stream>>>(
+        nb * N, used, scale, part, out);
+    if (int e = check_launch(ctx, "density_sum")) return e;
+  }
+  return 0;
 }
 
 }  // namespace qbh

@@ -994,6 +994,150 @@ k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 }
 
 // ------------------------------------------------------------------------------------
+// x pass of band sums of products of transforms, without a grid per band:
+//   part[range][d][r] = sum_s w_s Re (IM: Im) (conj(a_s(r)) b_{d,s}(r)),  d < NB
+// over a range of slots per blockIdx.y (w null: 1).  a and the b_d are y-transformed lines
+// (T2); a workgroup takes the NB + 1 fields of a slot one after the other through the same
+// row buffers, the next field's lines in flight, holds a(r) in registers and accumulates in
+// FP64.  Against storing the transforms as grids and multiplying them from memory (16 bytes a
+// point and band written and read, per field), MI355X: current
+// density of 128 bands at 72^3 2.90 -> 1.54 ms, of 64 bands at 60^3 1.19 -> 0.55; TD gradient of
+// 64 Si atoms, two steps, 103 -> 87 ms.  Bound like k_xpass2 by vector issue; at two waves per
+// SIMD the longest edges with NB = 3 spill (110^3, 64 bands: 8.9 -> 3.0 ms all the same).
+struct CrossFields {
+  const cplx<double>* t2[4];  // a, b_0 .. b_{NB-1}
+};
+template <int N1, int N2, int GPW, int NB, bool IM>
+__global__ void __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu(2)))
+k_xcross2(GridDev g, CrossFields fields, int nslots, int slots_per_wg,
+          const double* __restrict__ w, double* __restrict__ part) {
+  using C = cplx<double>;
+  constexpr int LPW = x_rows(N1, N2), YB = LPW * NWAVE, n = N1 * N2;
+  constexpr int TA = LPW * N2, TB = LPW * N1;
+  static_assert(TA <= 64 && TB <= 64, "one task per lane and stage");
+  using PD = Pad<N1, N2, QBH_XLDS_PAD>;
+  constexpr int LD = PD::row(n), S = N2 + PD::P;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int np1 = g.np1, np2 = g.np2, nlx = g.nlx;
+  C* tw = reinterpret_cast<C*>(smem_raw);
+  C* rows = tw + n;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  C* buf = rows + wave * LPW * LD;
+  const int nyb = (np1 + YB - 1) / YB;
+  const int z = blockIdx.x / nyb;
+  const int ywg = (blockIdx.x % nyb) * YB;
+  const int y0 = ywg + wave * LPW;
+  const int nyl = min(LPW, np1 - y0);
+  const int s0 = blockIdx.y * slots_per_wg;
+  const int s1 = min(nslots, s0 + slots_per_wg);
+  for (int i = threadIdx.x; i < n; i += NTHR) tw[i] = g.tw64[0][i];
+
+  // line elements of this thread, and the row positions outside the lines that stage A reads
+  // and that are cleared per field (see k_xpass2)
+  const long sstride = (long)np2 * nlx * np1;
+  constexpr int DUMP = YB * LD;
+  int lofs[GPW], gofs[GPW];
+#pragma unroll
+  for (int k = 0; k < GPW; ++k) {
+    const int q = threadIdx.x + k * NTHR;
+    const int dy = q % YB, lx = q / YB;
+    const bool in = q < nlx * YB;
+    lofs[k] = in ? dy * LD + PD::idx(g.line_x[lx]) : DUMP + (int)threadIdx.x;
+    gofs[k] = in && ywg + dy < np1 ? (z * nlx + lx) * np1 + ywg + dy : 0;
+  }
+  const int ja = g.xpos_max / N2 + 1;
+  const int jb = g.xneg_min / N2 - 1;
+  const int z0a = g.xpos_max + 1, z0b = min(N2 * ja, g.xneg_min);
+  const int z1a = max(N2 * (jb + 1), z0b), z1b = g.xneg_min;
+  const int nz0 = max(0, z0b - z0a), nz = nz0 + max(0, z1b - z1a);
+  constexpr int ZK = (LPW * 2 * N2 + 63) / 64;
+  int zofs[ZK];
+#pragma unroll
+  for (int k = 0; k < ZK; ++k) {
+    const int i = lane + 64 * k;
+    zofs[k] = -1;
+    if (i < LPW * nz) {
+      const int r = i / nz, j = i % nz;
+      zofs[k] = r * LD + PD::idx(j < nz0 ? z0a + j : z1a + j - nz0);
+    }
+  }
+  C pf[GPW];
+  auto prefetch = [&](const C* t2, int s) {
+    const C* src = t2 + s * sstride;
+#pragma unroll
+    for (int k = 0; k < GPW; ++k) {
+      const C e = src[gofs[k]];
+      pf[k].x = e.x;
+      pf[k].y = e.y;
+    }
+  };
+  // transforms the field in pf, prefetching the next; out: its values at x = k1 + N1 k2
+  const int rb = lane / N1, k1 = lane % N1;
+  auto transform = [&](const C* next, int snext, C(&out)[N2]) {
+#pragma unroll
+    for (int k = 0; k < ZK; ++k)
+      if (zofs[k] >= 0) buf[zofs[k]] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < GPW; ++k) rows[lofs[k]] = C{pf[k].x, pf[k].y};
+    __syncthreads();
+    if (next) prefetch(next, snext);
+    if (lane < TA) {
+      const int j2 = lane % N2;
+      C* row = buf + (lane / N2) * LD + j2;
+      C a[N1];
+#pragma unroll
+      for (int j1 = 0; j1 < N1; ++j1)
+        a[j1] = (j1 < ja || j1 > jb) ? row[S * j1] : C{0.0, 0.0};
+      sdft<N1, +1>(a);
+      twiddle_row<N1, +1>(a, tw, j2);
+#pragma unroll
+      for (int j1 = 0; j1 < N1; ++j1) row[S * j1] = a[j1];
+    }
+    wave_sync();
+    if (lane < TB) {
+      const C* blk = buf + rb * LD + S * k1;
+#pragma unroll
+      for (int j2 = 0; j2 < N2; ++j2) out[j2] = blk[j2];
+      sdft<N2, +1>(out);
+    }
+    __syncthreads();  // the next scatter overwrites rows read above
+  };
+
+  double acc[NB][N2];
+#pragma unroll
+  for (int d = 0; d < NB; ++d)
+#pragma unroll
+    for (int k2 = 0; k2 < N2; ++k2) acc[d][k2] = 0.0;
+  if (s0 < s1) prefetch(fields.t2[0], s0);
+  __syncthreads();
+  for (int s = s0; s < s1; ++s) {
+    C a[N2], b[N2];
+    transform(fields.t2[1], s, a);
+    const double ws = w ? w[s] : 1.0;
+#pragma unroll
+    for (int d = 0; d < NB; ++d) {
+      const bool last = d + 1 == NB;
+      transform(last ? (s + 1 < s1 ? fields.t2[0] : nullptr) : fields.t2[d + 2 < 4 ? d + 2 : 0],
+                last ? s + 1 : s, b);
+      if (lane < TB) {
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2)
+          acc[d][k2] += ws * (IM ? a[k2].x * b[k2].y - a[k2].y * b[k2].x
+                                 : a[k2].x * b[k2].x + a[k2].y * b[k2].y);
+      }
+    }
+  }
+  if (lane < TB && rb < nyl) {
+    const long N = (long)n * np1 * np2;
+    double* o = part + (long)blockIdx.y * NB * N + ((long)z * np1 + y0 + rb) * n + k1;
+#pragma unroll
+    for (int d = 0; d < NB; ++d)
+#pragma unroll
+      for (int k2 = 0; k2 < N2; ++k2) o[d * N + N1 * k2] = acc[d][k2];
+  }
+}
+
+// ------------------------------------------------------------------------------------
 // z pass, forward: T1 columns -> z transform (exp(-i)) -> x 1/N -> unpack -> output.
 // store 0: out[n][G] = ((out + add32) + kin[G]*psi[n][G]) + value;
 // store 1: out[n][G] = value;
@@ -1152,13 +1296,15 @@ k_zpass_fwd(GridDev g, const cplx<T>* __restrict__ t1, const double* __restrict_
 }
 
 // ------------------------------------------------------------------------------------
-// rho += sum of the nparts partial grids, in slot order (bound by HBM: nparts + 2 grids)
+// rho += scale * (sum of the nparts partial grids, in slot order; bound by HBM: nparts + 2
+// grids)
 template <int U>
 __global__ void __launch_bounds__(NTHR)
-k_density_sum(long N, int nparts, const double* __restrict__ part, double* __restrict__ rho) {
+k_density_sum(long N, int nparts, double scale, const double* __restrict__ part,
+              double* __restrict__ rho) {
   const long i = blockIdx.x * (long)NTHR + threadIdx.x;
   if (i >= N) return;
-  double r = rho[i];
+  double r = 0.0;
   int p = 0;
   for (; p + U <= nparts; p += U) {  // U partials in flight together
     double v[U];
@@ -1168,7 +1314,7 @@ k_density_sum(long N, int nparts, const double* __restrict__ part, double* __res
     for (int u = 0; u < U; ++u) r += v[u];
   }
   for (; p < nparts; ++p) r += part[p * N + i];
-  rho[i] = r;
+  rho[i] += scale * r;
 }
 
 // ------------------------------------------------------------------------------------
@@ -1192,6 +1338,9 @@ struct EdgeOps {
   // register x pass of the forward transform, from a complex or (scaled) real grid
   void (*xload)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
                 const double* f, bool real_input, double scale);
+  // band sums of products (FP64): nb fields b of 1 (real part) or 3 (imaginary part)
+  void (*xcross)(hipStream_t st, const GridDev& g, const CrossFields& fields, int nslots, int spw,
+                 int nb, const double* w, double* part);
 };
 
 // register-transform edges compiled by unit `part` (qbh_fft_edges.hip)
@@ -1293,6 +1442,25 @@ void launch_xload2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int 
     k_xload2<T, false, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
 }
 
+template <int N1, int N2>
+void launch_xcross2(hipStream_t st, const GridDev& g, const CrossFields& fields, int nslots,
+                    int spw, int nb, const double* w, double* part) {
+  constexpr int n = N1 * N2, YB = x_rows(N1, N2) * NWAVE;
+  constexpr int GS = x_short(n, YB), GF = (YB * n + NTHR - 1) / NTHR;
+  const dim3 grid(g.np2 * ((g.np1 + YB - 1) / YB), (nslots + spw - 1) / spw);
+  const size_t lds =
+      sizeof(cplx<double>) * ((size_t)n + (size_t)YB * Pad<N1, N2, QBH_XLDS_PAD>::row(n) + NTHR);
+  const bool small = (g.nlx * YB + NTHR - 1) / NTHR <= GS;
+  if (nb == 1 && small)
+    k_xcross2<N1, N2, GS, 1, false><<<grid, NTHR, lds, st>>>(g, fields, nslots, spw, w, part);
+  else if (nb == 1)
+    k_xcross2<N1, N2, GF, 1, false><<<grid, NTHR, lds, st>>>(g, fields, nslots, spw, w, part);
+  else if (small)
+    k_xcross2<N1, N2, GS, 3, true><<<grid, NTHR, lds, st>>>(g, fields, nslots, spw, w, part);
+  else
+    k_xcross2<N1, N2, GF, 3, true><<<grid, NTHR, lds, st>>>(g, fields, nslots, spw, w, part);
+}
+
 template <typename T, int N1, int N2>
 constexpr EdgeOps make_edge() {
   return EdgeOps{N1 * N2,
@@ -1304,7 +1472,8 @@ constexpr EdgeOps make_edge() {
                  launch_x2<T, X_VMUL, N1, N2>,
                  launch_x2<T, X_STORE, N1, N2>,
                  launch_x2<T, X_DENSITY, N1, N2>,
-                 launch_xload2<T, N1, N2>};
+                 launch_xload2<T, N1, N2>,
+                 sizeof(T) == 8 ? launch_xcross2<N1, N2> : nullptr};
 }
 
 }  // namespace qbh

@@ -174,6 +174,14 @@ int pipeline_x_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, 
                     double scale);
 int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* facs,
                        double* rho);
+// Band sums of products of transforms, for the edges cross_edge() names (FP64):
+//   nb 1: out[r] += scale sum_n w_n Re(conj(a_n(r)) b_n(r))
+//   nb 3: out[d N + r] += scale sum_n w_n Im(conj(a_n(r)) b_{d,n}(r))
+// a and the nb fields b are nbands coefficient columns each (leading dimensions lda, ldb), w
+// (device, nullable = 1) one weight per band
+bool cross_edge(const Basis* b);
+int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* const* bs,
+                   long ldb, int nbands, int nb, const double* w, double scale, double* out);
 size_t slot_bytes(const Basis* b, int prec);
 // Slot ranges of the density x pass for chunks of nslots slots: each workgroup sums all slots
 // of its rows, so the rows alone give np2 * np1 / rows-per-workgroup workgroups (216 at 72^3,

@@ -92,22 +92,24 @@ extern "C" int qbh_current(qbh_basis basis, const double* psi_dev, long ld, int 
   if (ld < g.ngw) return ofail(c, QBH_ERR_ARG, "ld < ngw");
   const long N = (long)g.np0 * g.np1 * g.np2;
   const int ngw = g.ngw;
-  // bands per chunk: four complex grids per band, about 1 GiB of grids per chunk
-  const int nb = (int)std::max(1L, std::min((long)nst, (1L << 30) / (64L * N)));
+  // bands per chunk: three scaled copies of their coefficients where the x pass forms the
+  // products, four complex grids per band elsewhere; about 1 GiB per chunk
+  const bool fused = cross_edge(b);
+  const int nb = (int)std::max(1L, std::min((long)nst, (1L << 30) / (fused ? 48L * ngw : 64L * N)));
   const int nblk = 256;
   std::vector<double> fac(nst);
   for (int n = 0; n < nst; ++n) {
     const double f = weight / omega * occ[n];
     fac[n] = f > 0.0 ? f : 0.0;
   }
-  const size_t bytes = sizeof(double) * (2 * 4 * (size_t)nb * N + 2 * 3 * (size_t)nb * ngw +
+  const size_t bytes = sizeof(double) * ((fused ? 0 : 2 * 4 * (size_t)nb * N) + 2 * 3 * (size_t)nb * ngw +
                                          (j_dev ? 0 : 3 * (size_t)N) + nst + 3 * nblk);
   double* buf = nullptr;
   if (hipMalloc(&buf, bytes) != hipSuccess)
     return ofail(c, QBH_ERR_ALLOC, "current scratch allocation failed");
   double* f0 = buf;
   double* fd = f0 + 2 * (size_t)nb * N;
-  double* ikc = fd + 2 * 3 * (size_t)nb * N;
+  double* ikc = fused ? buf : fd + 2 * 3 * (size_t)nb * N;
   double* jj = ikc + 2 * 3 * (size_t)nb * ngw;
   double* dfac = jj + (j_dev ? 0 : 3 * (size_t)N);
   double* part = dfac + nst;
@@ -122,6 +124,11 @@ extern "C" int qbh_current(qbh_basis basis, const double* psi_dev, long ld, int 
     const double* cp = psi_dev + 2 * (size_t)ld * n0;
     k_ikc<<<(unsigned)(((long)ngw * m + 255) / 256), 256, 0, c->stream>>>(ngw, m, b->kpgx, cp, ld,
                                                                           ikc);
+    if (fused) {
+      const double* fields[3] = {ikc, ikc + 2 * (size_t)m * ngw, ikc + 4 * (size_t)m * ngw};
+      r = pipeline_cross(c, b, cp, ld, fields, ngw, m, 3, dfac + n0, -1.0, jj);
+      continue;
+    }
     r = qbh_fft_backward(basis, cp, ld, m, 0, f0, 0);
     for (int d = 0; d < 3 && r == QBH_OK; ++d)
       r = qbh_fft_backward(basis, ikc + 2 * (size_t)d * m * ngw, ngw, m, 0,

@@ -425,9 +425,7 @@ static int cross(qbh_td_s* t, const double* zk, const double* u, const double* A
     k_sum_slices<<<nb256(R8 * C), 256, 0, cx->stream>>>(R8 * C, t->nsl, t->fsl, out);
     return true;
   };
-  const int nb = t->nb_cross;
-  double* fz = t->grids;
-  double* fU = t->grids + 2 * (size_t)nb * t->N;
+  const int nb = t->nb_cross;  // 0: the x pass forms the products
   // U_k = sum_m alpha_{k+m+1} u_m for every k (order blocks, like zk)
   for (int k = 0; k < o; ++k) {
     Combo cb{};
@@ -446,12 +444,23 @@ static int cross(qbh_td_s* t, const double* zk, const double* u, const double* A
                                                t->part);
     k_final<<<1, 256, 0, cx->stream>>>(NBLK, 3, t->part, -2.0, 1, gA3);
   }
+  // the order blocks are consecutive columns, of z_k as of U_k
+  const int cols = o * t->nst;
+  k_crossk_part<<<NBLK, 256, 0, cx->stream>>>(t->ngw, cols, t->h->b->kpgx, A[0], A[1], A[2], zk,
+                                             t->ubuf, t->part);
+  k_final<<<1, 256, 0, cx->stream>>>(NBLK, 3, t->part, -2.0, 1, gA3);
+  if (nb == 0) {
+    const double* U = t->ubuf;
+    if (int r = pipeline_cross(cx, h->b, zk, t->ngw, &U, t->ngw, cols, 1, nullptr,
+                               2.0 / (double)t->N, mu))
+      return r;
+    return tcheck(cx, "td cross");
+  }
+  double* fz = t->grids;
+  double* fU = t->grids + 2 * (size_t)nb * t->N;
   for (int k = 0; k < o; ++k) {
     const double* z = zk + k * B;
     const double* U = t->ubuf + k * B;
-    k_crossk_part<<<NBLK, 256, 0, cx->stream>>>(t->ngw, t->nst, t->h->b->kpgx, A[0], A[1], A[2],
-                                               z, U, t->part);
-    k_final<<<1, 256, 0, cx->stream>>>(NBLK, 3, t->part, -2.0, 1, gA3);
     for (int b0 = 0; b0 < t->nst; b0 += nb) {
       const int m = std::min(nb, t->nst - b0);
       if (int r = qbh_fft_backward(hb, z + 2 * (size_t)b0 * t->ngw, t->ngw, m, 0, fz, 0)) return r;
@@ -501,7 +510,10 @@ static int ensure_memory(qbh_td_s* t) {
   const size_t N = t->N;
   const int nck = (t->nsteps + t->ckpt - 1) / t->ckpt;
   // bands per transform chunk of the gradient products: two complex grids per band
-  t->nb_cross = (int)std::max<long>(1, std::min<long>(t->nst, (1L << 30) / (32L * (long)N)));
+  // (none at the edges whose x pass forms the products)
+  t->nb_cross = cross_edge(t->h->b)
+                    ? 0
+                    : (int)std::max<long>(1, std::min<long>(t->nst, (1L << 30) / (32L * (long)N)));
   size_t need = 0;
   auto add = [&](size_t d) { need += ((d * sizeof(double) + 255) / 256) * 256; };
   const size_t sizes[] = {(size_t)t->nst, 2 * (size_t)NBLK * 3, 2 * (size_t)(t->nsteps + 1),

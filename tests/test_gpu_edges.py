@@ -141,3 +141,45 @@ def test_density_slot_ranges(real, nb, grid):
             assert rel_err(rho.cpu().numpy() - start, ref) <= tol * 10  # start is ~10x ref
         basis.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("real,nb", [(False, 1), (False, 7), (False, 26), (True, 5)])
+@pytest.mark.parametrize("grid", [(24, 36, 30), (44, 18, 40), (64, 42, 20), (72, 20, 36),
+                                  (140, 24, 18), (22, 24, 18)])
+def test_current_edges(real, nb, grid):
+    """The current density (band sums of products of transforms), bands with no weight among
+    them, in one chunk and in chunks of a few bands, against the oracle's transforms."""
+    import torch
+    from oracle import fft as offt
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Context
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=25.0, nbands=nb, seed=27, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), *grid)
+    occ = np.where(np.arange(nb) % 4 == 2, 0.0, 1.0 + 0.05 * np.arange(nb))
+    ref = np.zeros((3, int(np.prod(grid))))
+    size = np.zeros(3)
+    for n in range(nb):
+        f0 = offt.backward(maps, sysm.psi[:, n]).ravel()
+        for d in range(3):
+            fd = offt.backward(maps, 1j * sysm.kpg[:, d] * sysm.psi[:, n]).ravel()
+            ref[d] -= occ[n] / sysm.omega * (np.conj(f0) * fd).imag
+            size[d] += occ[n] / sysm.omega * np.linalg.norm(np.abs(f0) * np.abs(fd))
+    r = sysm.rods
+    cd = to_dev(sysm.psi)
+    for cap in (8 << 30, 4 << 20):
+        ctx = Context(0, None)
+        ctx.set_workspace_cap(cap)
+        basis = Basis(ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+        j = torch.full((3, basis.N), np.nan, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        total = basis.current(cd.data_ptr(), basis.ngw, nb, occ, 1.0, sysm.omega,
+                              j_ptr=j.data_ptr())
+        ctx.sync()
+        got = j.cpu().numpy()
+        for d in range(3):
+            assert np.linalg.norm(got[d] - ref[d]) <= 1e-13 * size[d]
+            assert abs(total[d] - sysm.omega / basis.N * ref[d].sum()) <= \
+                1e-13 * sysm.omega / basis.N * size[d] * np.sqrt(basis.N)
+        basis.close()
+        ctx.close()
