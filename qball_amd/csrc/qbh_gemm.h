@@ -22,4 +22,16 @@ int mfma_gemm_qq(hipStream_t st, bool fp32, int R, int C, long Q, const void* X,
 int mfma_gemm_qc(hipStream_t st, bool fp32, int R, int C, long Q, const void* X, long ldx,
                  const void* Y, long ldy, void* O, long ldo, bool accumulate);
 
+// FP64, lower triangle (r >= c) of the symmetric product, whole tiles of it:
+// O_s[r + c R] = sum_{q in slice s} X[q + r ldx] X[q + c ldx], s < slices (as mfma_gemm_qq; the
+// count from mfma_sym_slices).
+int mfma_sym_slices(int R, long Q);
+int mfma_gemm_sym(hipStream_t st, int R, long Q, const double* X, long ldx, double* O, int slices,
+                  long ostride);
+
+// FP64, X lower triangular (zero above its diagonal): O[c + r ldo] = sum_{q <= r} X[q + r ldx]
+// Y[c + q ldy], q < R (as mfma_gemm_qc without the zero half of the reduction; O apart from Y).
+int mfma_gemm_tri(hipStream_t st, int R, int C, const double* X, long ldx, const double* Y,
+                  long ldy, double* O, long ldo);
+
 }  // namespace qbh

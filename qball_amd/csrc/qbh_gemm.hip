@@ -118,7 +118,29 @@ struct Args {
   int nblocks;   // tiles_r * tiles_c * slices (the grid is padded to a multiple of 8)
   int r_fastest; // consecutive blocks of one XCD step along r (else along c)
   int accumulate;
+  int lower;     // only the tiles on and below the diagonal (R = C)
+  int tri_q;     // X is lower triangular (R = Q): row r takes the reduction up to q = r only
 };
+
+// slice and tile of work item wid
+__device__ inline void tile_of(const Args& a, int wid, int& s, int& tr, int& tc) {
+  const int tiles = a.lower ? a.tiles_r * (a.tiles_r + 1) / 2 : a.tiles_r * a.tiles_c;
+  s = wid / tiles;
+  const int t = wid - s * tiles;
+  if (a.lower) {  // t = tr (tr + 1) / 2 + tc
+    tr = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+    while ((tr + 1) * (tr + 2) / 2 <= t) ++tr;
+    while (tr * (tr + 1) / 2 > t) --tr;
+    tc = t - tr * (tr + 1) / 2;
+  } else if (a.r_fastest) {
+    tr = t % a.tiles_r;
+    tc = t / a.tiles_r;
+    if (a.tri_q) tr = a.tiles_r - 1 - tr;  // the longest reductions first
+  } else {
+    tc = t % a.tiles_c;
+    tr = t / a.tiles_c;
+  }
+}
 
 // zeros that out-of-range lanes load instead of operand elements
 __device__ __attribute__((aligned(16))) double g_gemm_zero[2] = {0.0, 0.0};
@@ -216,20 +238,11 @@ __global__ void __launch_bounds__(kThreads, TB == 4 ? Mf<T>::WPE : KS > 1 ? 2 : 
   const int bid = blockIdx.x;
   const int wid = (bid & 7) * nb8 + (bid >> 3);
   if (wid >= a.nblocks) return;
-  const int tiles = a.tiles_r * a.tiles_c;
-  const int s = wid / tiles;
-  const int t = wid - s * tiles;
-  int tr, tc;
-  if (a.r_fastest) {
-    tr = t % a.tiles_r;
-    tc = t / a.tiles_r;
-  } else {
-    tc = t % a.tiles_c;
-    tr = t / a.tiles_c;
-  }
+  int s, tr, tc;
+  tile_of(a, wid, s, tr, tc);
   const int r0 = tr * BT, c0 = tc * BT;
   const long q0 = (long)s * a.qslice;
-  const long q1 = min(a.Q, q0 + a.qslice);
+  const long q1 = min(a.tri_q ? min(a.Q, (long)r0 + BT) : a.Q, q0 + a.qslice);
 
   const T* __restrict__ X = static_cast<const T*>(a.X);
   const T* __restrict__ Y = static_cast<const T*>(a.Y);
@@ -439,20 +452,11 @@ __global__ void __launch_bounds__(kThreads, TB == 4 ? 2 : 4) k_gemm_direct(Args 
   const int bid = blockIdx.x;
   const int wid = (bid & 7) * nb8 + (bid >> 3);
   if (wid >= a.nblocks) return;
-  const int tiles = a.tiles_r * a.tiles_c;
-  const int s = wid / tiles;
-  const int t = wid - s * tiles;
-  int tr, tc;
-  if (a.r_fastest) {
-    tr = t % a.tiles_r;
-    tc = t / a.tiles_r;
-  } else {
-    tc = t % a.tiles_c;
-    tr = t / a.tiles_c;
-  }
+  int s, tr, tc;
+  tile_of(a, wid, s, tr, tc);
   const int r0 = tr * 32 * TB, c0 = tc * 32 * TB;
   const long q0 = (long)s * a.qslice;
-  const long q1 = min(a.Q, q0 + a.qslice);
+  const long q1 = min(a.tri_q ? min(a.Q, (long)r0 + 32 * TB) : a.Q, q0 + a.qslice);
   const T* __restrict__ X = static_cast<const T*>(a.X);
   const T* __restrict__ Y = static_cast<const T*>(a.Y);
   const int tid = threadIdx.x;
@@ -600,7 +604,7 @@ void launch(Args a, hipStream_t st, int slices) {
   constexpr int KS = TB == 1 ? 2 : 1;
   a.tiles_r = (a.R + BT - 1) / BT;
   a.tiles_c = (a.C + BT - 1) / BT;
-  a.nblocks = a.tiles_r * a.tiles_c * slices;
+  a.nblocks = (a.lower ? a.tiles_r * (a.tiles_r + 1) / 2 : a.tiles_r * a.tiles_c) * slices;
   const unsigned grid = (unsigned)((a.nblocks + 7) / 8 * 8);
   // pairs are aligned vectors, and a pair never straddles the end of the range, when the
   // leading dimension and the range along the pair (Q for q-contiguous reads, C for
@@ -733,6 +737,55 @@ int mfma_gemm_qc(hipStream_t st, bool fp32, int R, int C, long Q, const void* X,
   a.r_fastest = 1;
   a.accumulate = accumulate ? 1 : 0;
   launch<true, true>(a, st, fp32, 1, best_tile(fp32 ? FORM_LDS32 : FORM_DIRECT64, R, C, Q, 1));
+  return 0;
+}
+
+// slices of the symmetric product: from eight 128 x 128 tiles on, as many as one round of two
+// workgroups per CU takes (1024 bands: 36 tiles, 14 slices, 504 workgroups), the rule of the F
+// product for fewer
+int mfma_sym_slices(int R, long Q) {
+  const long tr = (R + 127) / 128, low = tr * (tr + 1) / 2;
+  long s = low >= 8 ? std::max<long>(1, std::min<long>(512 / low, Q / 512))
+                    : tiling(false, R, R, Q).slices;
+  const long qs = mfma_slice_len(Q, (int)s);
+  return (int)((Q + qs - 1) / qs);
+}
+
+int mfma_gemm_sym(hipStream_t st, int R, long Q, const double* X, long ldx, double* O, int slices,
+                  long ostride) {
+  if (R <= 0 || Q <= 0 || slices <= 0) return -1;
+  Args a{};
+  a.R = a.C = R;
+  a.Q = Q;
+  a.X = a.Y = X;
+  a.ldx = a.ldy = ldx;
+  a.O = O;
+  a.ldo = R;
+  a.qslice = mfma_slice_len(Q, slices);
+  if ((Q + a.qslice - 1) / a.qslice != slices) return -1;
+  a.ostride = ostride;
+  a.lower = 1;
+  launch<false, false>(a, st, false, slices, best_tile(FORM_LDS64, R, R, Q, slices));
+  return 0;
+}
+
+int mfma_gemm_tri(hipStream_t st, int R, int C, const double* X, long ldx, const double* Y,
+                  long ldy, double* O, long ldo) {
+  if (R <= 0 || C <= 0) return -1;
+  Args a{};
+  a.R = R;
+  a.C = C;
+  a.Q = R;
+  a.X = X;
+  a.ldx = ldx;
+  a.Y = Y;
+  a.ldy = ldy;
+  a.O = O;
+  a.ldo = ldo;
+  a.qslice = ((long)R + kBQ - 1) / kBQ * kBQ;
+  a.r_fastest = 1;
+  a.tri_q = 1;
+  launch<true, true>(a, st, false, 1, best_tile(FORM_DIRECT64, R, C, R, 1));
   return 0;
 }
 
