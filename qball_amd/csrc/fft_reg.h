@@ -10,6 +10,7 @@
 // otherwise (9 = 3*3, 16 = 4*4).
 #pragma once
 #include "fft_device.h"
+#include "qbh_fft_edges.h"
 
 namespace qbh {
 
@@ -124,6 +125,74 @@ __device__ __forceinline__ void sdft(cplx<T>* a) {
   }
 }
 
+// FP32 transforms in the radix order of the Stockham passes (n = N1*N2 an F length): the first
+// stage is a chain of the plan's leading radices with their twiddles W_N1^e = W_n^{e N2} read
+// from the table tw of length n, the second the last radix, and each twiddle product stands
+// right before the radix it feeds, as in those passes, and rounds as theirs do (cmul_fused).
+template <typename T, int N1, int N2> constexpr bool stockham_order() {
+  return sizeof(T) == 4 && stockham_length(N1 * N2);
+}
+
+// a * w (DIR < 0: a * conj w) with the fused operations that the compiler makes of the
+// Stockham passes' cmul; left to itself it fuses some products of the unrolled chains the
+// other way round.
+template <int DIR>
+__device__ __forceinline__ cplx<float> cmul_fused(cplx<float> a, cplx<float> w) {
+  if (DIR < 0) w.y = -w.y;
+  return {fmaf(a.x, w.x, -(a.y * w.y)), fmaf(a.y, w.x, a.x * w.y)};
+}
+
+// length A*B as radix A then B (Cooley-Tukey, see ct), twiddles tw[e * stride]
+template <int A, int B, int DIR, typename T>
+__device__ __forceinline__ void ct_tab(cplx<T>* x, const cplx<T>* tw, int stride) {
+  cplx<T> m[B][A];
+#pragma unroll
+  for (int j2 = 0; j2 < B; ++j2) {
+#pragma unroll
+    for (int j1 = 0; j1 < A; ++j1) m[j2][j1] = x[j2 + B * j1];
+    dft<A, DIR>(m[j2]);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < A; ++k1) {
+    cplx<T> col[B];
+#pragma unroll
+    for (int j2 = 0; j2 < B; ++j2) {
+      col[j2] = m[j2][k1];
+      if (j2 > 0) {
+        col[j2] = cmul_fused<DIR>(col[j2], tw[j2 * k1 * stride]);
+      }
+    }
+    dft<B, DIR>(col);
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) x[k1 + A * k2] = col[k2];
+  }
+}
+
+// first-stage DFT of length N1 of a transform of length N1*N2 (twiddle table tw)
+template <int N1, int N2, int DIR, typename T>
+__device__ __forceinline__ void stage_a(cplx<T>* a, const cplx<T>* tw) {
+  if constexpr (!stockham_order<T, N1, N2>()) {
+    sdft<N1, DIR>(a);
+  } else if constexpr (N1 == 4 || N1 == 8) {
+    dft<N1, DIR>(a);
+  } else if constexpr (N1 == 12 || N1 == 16) {
+    ct_tab<4, N1 / 4, DIR>(a, tw, N2);
+  } else {
+    static_assert(N1 == 6 || N1 == 10 || N1 == 14, "no Stockham chain");
+    ct_tab<2, N1 / 2, DIR>(a, tw, N2);
+  }
+}
+
+// second-stage DFT of length N2 at k1 of the first stage (F forms: with the stage twiddles)
+template <int N1, int N2, int DIR, typename T>
+__device__ __forceinline__ void stage_b(cplx<T>* b, const cplx<T>* tw, int k1) {
+  if constexpr (stockham_order<T, N1, N2>()) {
+#pragma unroll
+    for (int j2 = 1; j2 < N2; ++j2) b[j2] = cmul_fused<DIR>(b[j2], tw[k1 * j2]);
+  }
+  sdft<N2, DIR>(b);
+}
+
 // a[k] *= W_n^{DIR e k}, k < K, n the length of the table tw (e (K - 1) < n).  FP64 reads every
 // power from the table: local Hψ is 1.2 to 1.9 times closer to 64-bit reference transforms
 // than with the repeated products of w = tw[e] that FP32 forms (140^3: 5.3e-16 against 8.2e-16
@@ -185,8 +254,8 @@ __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const 
       cplx<T> a[N1];
 #pragma unroll
       for (int j1 = 0; j1 < N1; ++j1) a[j1] = row[S * j1];
-      sdft<N1, DIR>(a);
-      twiddle_row<N1, DIR>(a, tw, j2);
+      stage_a<N1, N2, DIR>(a, tw);
+      if constexpr (!stockham_order<T, N1, N2>()) twiddle_row<N1, DIR>(a, tw, j2);
 #pragma unroll
       for (int k1 = 0; k1 < N1; ++k1) row[S * k1] = a[k1];
     }
@@ -201,7 +270,7 @@ __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const 
       const cplx<T>* blk = buf + r * ld + S * k1;
 #pragma unroll
       for (int j2 = 0; j2 < N2; ++j2) b[ib][j2] = blk[j2];
-      sdft<N2, DIR>(b[ib]);
+      stage_b<N1, N2, DIR>(b[ib], tw, k1);
     }
   }
   wave_sync();

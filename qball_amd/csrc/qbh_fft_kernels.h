@@ -645,7 +645,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   // 140 = 14*10: x pass 6.24 -> 6.01 ms per FP64 Hψ).  Not for the FP64 kernels with the
   // full line-element count, which have no registers to spare.
   constexpr int GS = x_short(n, YB);
-  constexpr bool TWB = QBH_XTWB && (sizeof(T) == 4 || GPW <= GS);
+  constexpr bool TWB = QBH_XTWB && (sizeof(T) == 4 || GPW <= GS) && !stockham_order<T, N1, N2>();
   cplx<T> twb[IB][TWB ? N2 - 1 : 1];
   if constexpr (TWB && OP == X_VMUL) {
 #pragma unroll
@@ -760,8 +760,8 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 #pragma unroll
         for (int j1 = 0; j1 < N1; ++j1)
           a[j1] = (j1 < ja || j1 > jb) ? row[S * j1] : cplx<T>{T(0), T(0)};
-        sdft<N1, +1>(a);
-        twiddle_row<N1, +1>(a, tw, j2);
+        stage_a<N1, N2, +1>(a, tw);
+        if constexpr (!stockham_order<T, N1, N2>()) twiddle_row<N1, +1>(a, tw, j2);
 #pragma unroll
         for (int k1 = 0; k1 < N1; ++k1) row[S * k1] = a[k1];
       }
@@ -780,7 +780,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
           const cplx<T>* blk = buf + r * LD + S * k1;
 #pragma unroll
           for (int j2 = 0; j2 < N2; ++j2) bs[ib][j2] = blk[j2];
-          sdft<N2, +1>(bs[ib]);
+          stage_b<N1, N2, +1>(bs[ib], tw, k1);
         }
       }
       wave_sync();
@@ -805,6 +805,44 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
       __syncthreads();  // the next scatter overwrites the rows read above
       return;
     }
+    if constexpr (OP == X_VMUL && stockham_order<T, N1, N2>()) {
+      // F forms: v psi(r) back into the rows in natural order, then the forward transform in
+      // the same radix order: one LDS round trip more than the transposed form below, whose
+      // reversed radix order rounds differently (110^3, 300 bands: x pass 1.66 -> 0.67 ms
+      // against the Stockham passes)
+      cplx<T> bs[IB][N2];
+#pragma unroll
+      for (int ib = 0; ib < IB; ++ib) {
+        const int t = lane + 64 * ib;
+        if (t < TB) {
+          const cplx<T>* blk = buf + (t / N1) * LD + S * (t % N1);
+#pragma unroll
+          for (int j2 = 0; j2 < N2; ++j2) bs[ib][j2] = blk[j2];
+          stage_b<N1, N2, +1>(bs[ib], tw, t % N1);
+        }
+      }
+      wave_sync();
+#pragma unroll
+      for (int ib = 0; ib < IB; ++ib) {
+        const int t = lane + 64 * ib;
+        if (t < TB) {
+          const int r = t / N1, k1 = t % N1;
+#pragma unroll
+          for (int k2 = 0; k2 < N2; ++k2)
+            buf[r * LD + PD::idx(k1 + N1 * k2)] = {vr[ib][k2] * bs[ib][k2].x,
+                                                   vr[ib][k2] * bs[ib][k2].y};
+        }
+      }
+      wave_sync();
+      rows_fft<N1, N2, LPW, -1, QBH_XLDS_PAD>(buf, LPW, LD, tw, lane);
+      __syncthreads();
+      cplx<T>* dst = t2 + s * sstride;
+#pragma unroll
+      for (int k = 0; k < GPW; ++k)
+        if ((gok >> k) & 1u) dst[gofs[k]] = rows[lofs[k]];
+      __syncthreads();
+      return;
+    }
     // stage B: backward DFT_N2 -> psi(r); multiply / accumulate; forward DFT_N2
     double f1 = 0, f2 = 0, b1 = 0, b2 = 0;
     if (OP == X_DENSITY) {
@@ -826,7 +864,7 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
         cplx<T> b[N2];
 #pragma unroll
         for (int j2 = 0; j2 < N2; ++j2) b[j2] = blk[j2];
-        sdft<N2, +1>(b);
+        stage_b<N1, N2, +1>(b, tw, k1);
         if (OP == X_VMUL) {
 #pragma unroll
           for (int k2 = 0; k2 < N2; ++k2) b[k2] = {vr[ib][k2] * b[k2].x, vr[ib][k2] * b[k2].y};

@@ -183,3 +183,44 @@ def test_current_edges(real, nb, grid):
                 1e-13 * sysm.omega / basis.N * size[d] * np.sqrt(basis.N)
         basis.close()
         ctx.close()
+
+
+@pytest.mark.parametrize("n", (18, 20, 24, 30, 42, 44, 56, 66, 70, 84, 88, 110, 112, 132, 154,
+                               176))
+@pytest.mark.parametrize("real", (True, False))
+def test_fp32_stockham_order(gpu_ctx, n, real):
+    """FP32 register transforms that keep the Stockham passes' radix order round like them:
+    backward, forward and local Hψ bit for bit, the edge along each axis."""
+    import torch
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    nb = 3
+    sysm = make_system(ncell=1, ecut_ry=12.0, nbands=nb, seed=31, complex_basis=not real)
+    r, cd = sysm.rods, to_dev(sysm.psi)
+    nslots = (nb + 1) // 2 if real else nb
+    rng = np.random.default_rng(n)
+    for axis in range(3):
+        grid = [22, 22, 22]  # (no register form)
+        grid[axis] = n
+        basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid,
+                      sysm.b)
+        vd = real_to_dev(rng.standard_normal(basis.N))
+        gd = real_to_dev(rng.standard_normal(2 * nslots * basis.N))
+        ham = Hamiltonian(gpu_ctx, basis)
+        ham.set_vloc(vd.data_ptr())
+        out = []
+        for reg in (1, 0):
+            ham.set_tuning("zy_reg", reg)
+            ham.set_tuning("x_reg", reg)
+            f = torch.zeros(2 * nslots * basis.N, dtype=torch.float64, device="cuda")
+            hd, back = torch.zeros_like(cd), torch.zeros_like(cd)
+            torch.cuda.synchronize()
+            basis.backward(cd.data_ptr(), basis.ngw, nb, real, f.data_ptr(), 0x10)
+            basis.forward(gd.data_ptr(), nb, real, back.data_ptr(), basis.ngw, 0x10)
+            ham.hpsi(cd.data_ptr(), basis.ngw, nb, sysm.occ, hd.data_ptr(), basis.ngw, flags=0x14)
+            gpu_ctx.sync()
+            out.append((f, back, hd))
+        for a, b in zip(*out):
+            assert torch.equal(a, b)
+        ham.close()
+        basis.close()
