@@ -496,10 +496,8 @@ int qbh::hpsi_impl(Ham* h, const double* psi, long ld, int nst, const double* oc
       a.mode = mode;
       a.wait_z = join;
       a.add32 = add32;
-      if (int r = pipeline_bwd_yz(c, b, a)) return r;
-      if (int r = pipeline_x_vmul(c, b, a, h->v)) return r;
-      return pipeline_fwd_zy_accumulate(c, b, a, hpsi, ldh, kin ? h->kin : nullptr,
-                                        z_overwrites ? 2 : 0);
+      return pipeline_vmul(c, b, a, h->v, hpsi, ldh, kin ? h->kin : nullptr,
+                           z_overwrites ? 2 : 0);
     });
     if (join) hipStreamWaitEvent(main, join, 0);  // also on early exit
     if (r) return r;

@@ -74,18 +74,34 @@ static const EdgeOps& zy_ops(const Basis* b, int n, int prec) {
   return r ? *r : kStockham[prec][n <= 144 ? 0 : 1];
 }
 
-int pipeline_bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a) {
+static int bwd_z(Ctx* ctx, Basis* b, const PipelineArgs& a) {
   const GridDev& g = b->g;
   {
     TimedLaunch tl(ctx, "zpass_bwd");
     zy_ops(b, g.np2, a.prec).zbwd(ctx->stream, g, a);
   }
-  if (int r = check_launch(ctx, "zpass_bwd")) return r;
+  return check_launch(ctx, "zpass_bwd");
+}
+
+int pipeline_bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a) {
+  const GridDev& g = b->g;
+  if (int r = bwd_z(ctx, b, a)) return r;
   {
     TimedLaunch tl(ctx, "ypass_bwd");
     zy_ops(b, g.np1, a.prec).ybwd(ctx->stream, g, a);
   }
   return check_launch(ctx, "ypass_bwd");
+}
+
+static int fwd_z(Ctx* ctx, Basis* b, const PipelineArgs& a, double* out, long ldo,
+                 const double* kin, int store) {
+  const GridDev& g = b->g;
+  if (a.wait_z) hipStreamWaitEvent(ctx->stream, a.wait_z, 0);
+  {
+    TimedLaunch tl(ctx, "zpass_fwd");
+    zy_ops(b, g.np2, a.prec).zfwd(ctx->stream, g, a, out, ldo, kin, store);
+  }
+  return check_launch(ctx, "zpass_fwd");
 }
 
 int pipeline_fwd_zy_accumulate(Ctx* ctx, Basis* b, const PipelineArgs& a, double* out, long ldo,
@@ -96,12 +112,7 @@ int pipeline_fwd_zy_accumulate(Ctx* ctx, Basis* b, const PipelineArgs& a, double
     zy_ops(b, g.np1, a.prec).yfwd(ctx->stream, g, a);
   }
   if (int r = check_launch(ctx, "ypass_fwd")) return r;
-  {
-    if (a.wait_z) hipStreamWaitEvent(ctx->stream, a.wait_z, 0);
-    TimedLaunch tl(ctx, "zpass_fwd");
-    zy_ops(b, g.np2, a.prec).zfwd(ctx->stream, g, a, out, ldo, kin, store);
-  }
-  return check_launch(ctx, "zpass_fwd");
+  return fwd_z(ctx, b, a, out, ldo, kin, store);
 }
 
 // slots per x-pass workgroup: keep >= 4096 workgroups in flight while amortising the
@@ -160,11 +171,42 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
   return check_launch(ctx, name);
 }
 
-int pipeline_x_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v) {
+static int x_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v) {
   return a.prec == PREC_FP64
              ? xpass_t<double, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul")
              : xpass_t<float, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul");
 }
+// plane form of local Hψ for this basis and precision, or null.  FP32 keeps the passes: the
+// plane's forward y transform has another radix order, which rounds differently.
+static const EdgeOps* plane_ops(const Basis* b, int prec) {
+  const GridDev& g = b->g;
+  if (prec != PREC_FP64 || g.np0 != g.np1 || !b->tune.zy_reg || !b->tune.x_reg) return nullptr;
+  const EdgeOps* r = register_ops(g.np0, prec);
+  return r && r->plane && r->plane_fits(g) ? r : nullptr;
+}
+
+int pipeline_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v, double* out,
+                  long ldo, const double* kin, int store) {
+  const GridDev& g = b->g;
+  if (const EdgeOps* r = plane_ops(b, a.prec)) {
+    if (int e = bwd_z(ctx, b, a)) return e;
+    // slots per workgroup: as many as leave 2048 workgroups (72^3, 128 complex bands: 1, 2, 4, 8
+    // slots 360, 330, 320, 346 us; 64^3, 128 real bands 108, 100, 98, 97)
+    int spw = 1;
+    while (spw < 16 && (long)g.np2 * ((a.nslots + 2 * spw - 1) / (2 * spw)) >= 2048) spw *= 2;
+    if (b->tune.x_spw > 0) spw = std::min(b->tune.x_spw, a.nslots);
+    {
+      TimedLaunch tl(ctx, "plane_vmul");
+      r->plane(ctx->stream, g, a, spw, v);
+    }
+    if (int e = check_launch(ctx, "plane_vmul")) return e;
+    return fwd_z(ctx, b, a, out, ldo, kin, store);
+  }
+  if (int e = pipeline_bwd_yz(ctx, b, a)) return e;
+  if (int e = x_vmul(ctx, b, a, v)) return e;
+  return pipeline_fwd_zy_accumulate(ctx, b, a, out, ldo, kin, store);
+}
+
 int pipeline_x_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f) {
   return a.prec == PREC_FP64
              ? xpass_t<double, X_STORE>(ctx, b, a, nullptr, f, nullptr, 1.0, 0, "xpass_store")

@@ -1379,6 +1379,10 @@ struct EdgeOps {
   // band sums of products (FP64): nb fields b of 1 (real part) or 3 (imaginary part)
   void (*xcross)(hipStream_t st, const GridDev& g, const CrossFields& fields, int nslots, int spw,
                  int nb, const double* w, double* part);
+  // y, x and y passes of Hψ in one kernel (FP64, both edges n): its LDS for nlx lines and
+  // launch (null for the edges whose plane never fits)
+  bool (*plane_fits)(const GridDev& g);
+  void (*plane)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw, const double* v);
 };
 
 // register-transform edges compiled by unit `part` (qbh_fft_edges.hip)
@@ -1499,6 +1503,10 @@ void launch_xcross2(hipStream_t st, const GridDev& g, const CrossFields& fields,
     k_xcross2<N1, N2, GF, 3, true><<<grid, NTHR, lds, st>>>(g, fields, nslots, spw, w, part);
 }
 
+}  // namespace qbh
+#include "qbh_fft_plane.h"
+namespace qbh {
+
 template <typename T, int N1, int N2>
 constexpr EdgeOps make_edge() {
   return EdgeOps{N1 * N2,
@@ -1511,7 +1519,9 @@ constexpr EdgeOps make_edge() {
                  launch_x2<T, X_STORE, N1, N2>,
                  launch_x2<T, X_DENSITY, N1, N2>,
                  launch_xload2<T, N1, N2>,
-                 sizeof(T) == 8 ? launch_xcross2<N1, N2> : nullptr};
+                 sizeof(T) == 8 ? launch_xcross2<N1, N2> : nullptr,
+                 PlaneOps<T, N1, N2>::fits(),
+                 PlaneOps<T, N1, N2>::launch()};
 }
 
 }  // namespace qbh

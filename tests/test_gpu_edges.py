@@ -224,3 +224,40 @@ def test_fp32_stockham_order(gpu_ctx, n, real):
             assert torch.equal(a, b)
         ham.close()
         basis.close()
+
+
+@pytest.mark.parametrize("n,np2,ecut,nb,real", [
+    (18, 20, 12.0, 1, True), (20, 18, 25.0, 3, False), (36, 30, 25.0, 6, True),
+    (44, 24, 25.0, 2, False), (48, 50, 170.0, 2, True), (60, 22, 25.0, 5, True),
+    (64, 30, 60.0, 3, False), (72, 36, 60.0, 67, True), (80, 20, 25.0, 4, False),
+    (84, 20, 25.0, 3, True), (88, 28, 60.0, 2, False), (108, 20, 25.0, 4, True)])
+def test_plane_vmul(gpu_ctx, n, np2, ecut, nb, real):
+    """Local Hψ on square cross-sections, whose y, x and y passes are one kernel: with one and
+    several slots per workgroup, the two workgroup sizes, spheres filling the plane (more
+    columns than are loaded ahead) and partly filled last row groups."""
+    import torch
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=ecut, nbands=nb, seed=41, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), n, n, np2)
+    r, c = sysm.rods, sysm.psi
+    basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"],
+                  (n, n, np2), sysm.b)
+    v = np.random.default_rng(n).standard_normal(basis.N)
+    vd, cd = real_to_dev(v), to_dev(c)
+    hd = torch.zeros_like(cd)
+    ham = Hamiltonian(gpu_ctx, basis)
+    ham.set_vloc(vd.data_ptr())
+    gpu_ctx.timing_report()
+    gpu_ctx.set_timing(True)
+    ham.hpsi(cd.data_ptr(), basis.ngw, nb, sysm.occ, hd.data_ptr(), basis.ngw, flags=0x4)
+    gpu_ctx.sync()
+    ran = gpu_ctx.timing_report()
+    gpu_ctx.set_timing(False)
+    assert "plane_vmul" in ran
+    ref = oh.rs_mul_add(maps, c, v, np.zeros_like(c))
+    assert rel_err(from_dev(hd, basis.ngw, nb), ref) <= 1e-12
+    ham.close()
+    basis.close()
