@@ -104,8 +104,7 @@ extern "C" int qbh_fft_backward(qbh_basis basis, const double* c_dev, long ld, i
     a.nst = nbands;
     a.band0 = pair ? 2 * s0 : s0;
     a.mode = mode;
-    if (int r = pipeline_bwd_yz(c, b, a)) return r;
-    return pipeline_x_store(c, b, a, f_dev + 2 * (long)s0 * N);
+    return pipeline_store(c, b, a, f_dev + 2 * (long)s0 * N);
   });
 }
 
@@ -172,8 +171,7 @@ extern "C" int qbh_fft_backward_noalloc(qbh_basis basis, const double* c_dev, lo
         a.nst = nbands;
         a.band0 = pair ? 2 * s0 : s0;
         a.mode = mode;
-        if (int r = pipeline_bwd_yz(c, b, a)) return r;
-        return pipeline_x_store(c, b, a, f_dev + 2 * (long)s0 * N);
+        return pipeline_store(c, b, a, f_dev + 2 * (long)s0 * N);
       },
       c->scratch, kNoallocScratchBytes);
 }
@@ -196,8 +194,7 @@ extern "C" int qbh_fft_forward(qbh_basis basis, const double* f_dev, int nbands,
     a.nst = nbands;
     a.band0 = pair ? 2 * s0 : s0;
     a.mode = mode;
-    if (int r = pipeline_x_load(c, b, a, f_dev + 2 * (long)s0 * N, 0, 1.0)) return r;
-    return pipeline_fwd_zy_accumulate(c, b, a, c_dev, ld, nullptr, 1);
+    return pipeline_load(c, b, a, f_dev + 2 * (long)s0 * N, 0, 1.0, c_dev, ld);
   });
 }
 
@@ -215,8 +212,7 @@ extern "C" int qbh_fft_forward_real(qbh_basis basis, const double* rho_dev, doub
     a.nst = 1;
     a.band0 = 0;
     a.mode = mode;
-    if (int r = pipeline_x_load(c, b, a, rho_dev, 1, scale)) return r;
-    return pipeline_fwd_zy_accumulate(c, b, a, c_dev, b->g.ngw, nullptr, 1);
+    return pipeline_load(c, b, a, rho_dev, 1, scale, c_dev, b->g.ngw);
   });
 }
 
@@ -577,7 +573,7 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
   // caller's workspace cap; without memory for them, one range)
   const size_t nfac = ((nst + 4 * (size_t)nslots + 31) / 32) * 32;
   const size_t chunk = std::max<size_t>(1, c->ws_cap / slot_bytes(b, prec));
-  int parts = density_parts(b, (int)std::min<size_t>(nslots, chunk), prec,
+  int parts = pipeline_density_parts(b, (int)std::min<size_t>(nslots, chunk), prec,
                             std::min<size_t>(c->ws_cap, size_t(256) << 20));
   double* dfac = nullptr;
   if (parts > 1)
@@ -600,8 +596,7 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
     k_dens_facs<<<(a.nslots + 255) / 256, 256, 0, c->stream>>>(a.nslots, a.band0, nst, pair ? 1 : 0,
                                                                dfac, psi_dev, ld,
                                                                slotf + 4 * (size_t)s0);
-    if (int r = pipeline_bwd_yz(c, b, a)) return r;
-    return pipeline_x_density(c, b, a, slotf + 4 * (size_t)s0, rho_dev);
+    return pipeline_density(c, b, a, slotf + 4 * (size_t)s0, rho_dev);
   });
   hipStreamSynchronize(c->stream);
   if (r) return r;

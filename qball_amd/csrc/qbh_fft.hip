@@ -61,7 +61,8 @@ static constexpr EdgeOps stockham_edge() {
                  nullptr,
                  nullptr,
                  nullptr,
-                 nullptr};
+                 nullptr,
+                 {}};
 }
 static const EdgeOps kStockham[2][2] = {
     {stockham_edge<double, 144>(), stockham_edge<double, 256>()},
@@ -83,7 +84,7 @@ static int bwd_z(Ctx* ctx, Basis* b, const PipelineArgs& a) {
   return check_launch(ctx, "zpass_bwd");
 }
 
-int pipeline_bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a) {
+static int bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a) {
   const GridDev& g = b->g;
   if (int r = bwd_z(ctx, b, a)) return r;
   {
@@ -104,8 +105,8 @@ static int fwd_z(Ctx* ctx, Basis* b, const PipelineArgs& a, double* out, long ld
   return check_launch(ctx, "zpass_fwd");
 }
 
-int pipeline_fwd_zy_accumulate(Ctx* ctx, Basis* b, const PipelineArgs& a, double* out, long ldo,
-                               const double* kin, int store) {
+static int fwd_zy(Ctx* ctx, Basis* b, const PipelineArgs& a, double* out, long ldo,
+                  const double* kin, int store) {
   const GridDev& g = b->g;
   {
     TimedLaunch tl(ctx, "ypass_fwd");
@@ -171,60 +172,84 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
   return check_launch(ctx, name);
 }
 
-static int x_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v) {
-  return a.prec == PREC_FP64
-             ? xpass_t<double, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul")
-             : xpass_t<float, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul");
-}
-// plane form of local Hψ for this basis and precision, or null.  FP32 keeps the passes: the
-// plane's forward y transform has another radix order, which rounds differently.
-static const EdgeOps* plane_ops(const Basis* b, int prec) {
+// plane forms for this basis and precision, or null.  FP32 keeps the passes: the plane's
+// forward y transform has another radix order, which rounds differently.
+static const PlaneOps* plane_ops(const Basis* b, int prec) {
   const GridDev& g = b->g;
   if (prec != PREC_FP64 || g.np0 != g.np1 || !b->tune.zy_reg || !b->tune.x_reg) return nullptr;
   const EdgeOps* r = register_ops(g.np0, prec);
-  return r && r->plane && r->plane_fits(g) ? r : nullptr;
+  return r && r->plane.fits && r->plane.fits(g) ? &r->plane : nullptr;
+}
+
+// slots per plane workgroup: as many as leave 2048 workgroups (72^3, 128 complex bands: 1, 2,
+// 4, 8 slots 360, 330, 320, 346 us; 64^3, 128 real bands 108, 100, 98, 97)
+static int plane_spw(const Basis* b, int nslots) {
+  if (b->tune.x_spw > 0) return std::min(b->tune.x_spw, nslots);
+  int spw = 1;
+  while (spw < 16 && (long)b->g.np2 * ((nslots + 2 * spw - 1) / (2 * spw)) >= 2048) spw *= 2;
+  return spw;
+}
+
+static int plane_pass(Ctx* ctx, Basis* b, const PipelineArgs& a, PlaneOps::Launch f, int spw,
+                      const double* in, double* out, const double* dens, int cplx_density,
+                      double scale, const char* name) {
+  {
+    TimedLaunch tl(ctx, name);
+    f(ctx->stream, b->g, a, spw, in, out, dens, cplx_density, scale);
+  }
+  return check_launch(ctx, name);
 }
 
 int pipeline_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v, double* out,
                   long ldo, const double* kin, int store) {
-  const GridDev& g = b->g;
-  if (const EdgeOps* r = plane_ops(b, a.prec)) {
+  if (const PlaneOps* p = plane_ops(b, a.prec)) {
     if (int e = bwd_z(ctx, b, a)) return e;
-    // slots per workgroup: as many as leave 2048 workgroups (72^3, 128 complex bands: 1, 2, 4, 8
-    // slots 360, 330, 320, 346 us; 64^3, 128 real bands 108, 100, 98, 97)
-    int spw = 1;
-    while (spw < 16 && (long)g.np2 * ((a.nslots + 2 * spw - 1) / (2 * spw)) >= 2048) spw *= 2;
-    if (b->tune.x_spw > 0) spw = std::min(b->tune.x_spw, a.nslots);
-    {
-      TimedLaunch tl(ctx, "plane_vmul");
-      r->plane(ctx->stream, g, a, spw, v);
-    }
-    if (int e = check_launch(ctx, "plane_vmul")) return e;
+    if (int e = plane_pass(ctx, b, a, p->vmul, plane_spw(b, a.nslots), v, nullptr, nullptr, 0, 1.0,
+                           "plane_vmul"))
+      return e;
     return fwd_z(ctx, b, a, out, ldo, kin, store);
   }
-  if (int e = pipeline_bwd_yz(ctx, b, a)) return e;
-  if (int e = x_vmul(ctx, b, a, v)) return e;
-  return pipeline_fwd_zy_accumulate(ctx, b, a, out, ldo, kin, store);
+  if (int e = bwd_yz(ctx, b, a)) return e;
+  const int e = a.prec == PREC_FP64
+      ? xpass_t<double, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul")
+      : xpass_t<float, X_VMUL>(ctx, b, a, v, nullptr, nullptr, 1.0, 0, "xpass_vmul");
+  return e ? e : fwd_zy(ctx, b, a, out, ldo, kin, store);
 }
 
-int pipeline_x_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f) {
+int pipeline_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f) {
+  if (const PlaneOps* p = plane_ops(b, a.prec); p && p->store) {
+    if (int e = bwd_z(ctx, b, a)) return e;
+    return plane_pass(ctx, b, a, p->store, plane_spw(b, a.nslots), nullptr, f, nullptr, 0, 1.0,
+                      "plane_store");
+  }
+  if (int e = bwd_yz(ctx, b, a)) return e;
   return a.prec == PREC_FP64
              ? xpass_t<double, X_STORE>(ctx, b, a, nullptr, f, nullptr, 1.0, 0, "xpass_store")
              : xpass_t<float, X_STORE>(ctx, b, a, nullptr, f, nullptr, 1.0, 0, "xpass_store");
 }
-int pipeline_x_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, int real_input,
-                    double scale) {
-  if (real_input)
-    return a.prec == PREC_FP64
-               ? xpass_t<double, X_LOAD_REAL>(ctx, b, a, f, nullptr, nullptr, scale, 0,
-                                              "xpass_load")
-               : xpass_t<float, X_LOAD_REAL>(ctx, b, a, f, nullptr, nullptr, scale, 0,
-                                             "xpass_load");
-  return a.prec == PREC_FP64
-             ? xpass_t<double, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load")
-             : xpass_t<float, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load");
+
+int pipeline_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, int real_input,
+                  double scale, double* out, long ldo) {
+  int e;
+  if (const PlaneOps* p = plane_ops(b, a.prec); p && p->load) {
+    e = plane_pass(ctx, b, a, real_input ? p->load_real : p->load, plane_spw(b, a.nslots), f,
+                   nullptr, nullptr, 0, scale, "plane_load");
+    return e ? e : fwd_z(ctx, b, a, out, ldo, nullptr, 1);
+  }
+  if (a.prec == PREC_FP64)
+    e = real_input ? xpass_t<double, X_LOAD_REAL>(ctx, b, a, f, nullptr, nullptr, scale, 0, "xpass_load")
+                   : xpass_t<double, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load");
+  else
+    e = real_input ? xpass_t<float, X_LOAD_REAL>(ctx, b, a, f, nullptr, nullptr, scale, 0, "xpass_load")
+                   : xpass_t<float, X_LOAD>(ctx, b, a, f, nullptr, nullptr, 1.0, 0, "xpass_load");
+  return e ? e : fwd_zy(ctx, b, a, out, ldo, nullptr, 1);
 }
-int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
+
+// Slot ranges of the density x pass for chunks of nslots slots: each workgroup sums all slots
+// of its rows, so the rows alone give np2 * np1 / rows-per-workgroup workgroups (216 at 72^3,
+// 1260 at 140^3: 2.5 rounds of two per CU).  Ranges for about 4096 workgroups, at least 4
+// slots each, with at most cap_bytes of partial grids.
+static int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
   const GridDev& g = b->g;
   const EdgeOps* r = b->tune.x_reg ? register_ops(g.np0, prec) : nullptr;
   const int yb = (r ? r->xr : prec == PREC_FP64 ? Cfg<double>::LPW : Cfg<float>::LPW) * NWAVE;
@@ -235,17 +260,46 @@ int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
   return (int)std::max<long>(p, 1);
 }
 
-int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* dens,
-                       double* rho) {
+// The same for the plane form, whose workgroups are few and long: of up to 16 ranges the number
+// with the fewest slots times rounds of resident workgroups, the smaller one if equal.  Density
+// without z passes, passes -> plane: 24^3, 16 real bands 23 -> 15 us; 64^3, 128 real bands 98 ->
+// 66; 72^3, 64 complex bands 136 -> 122; 88^3, 100 real bands 231 -> 196.
+static int plane_parts(const Basis* b, const PlaneOps* p, int nslots, size_t cap_bytes) {
+  const GridDev& g = b->g;
+  const size_t grid = 8 * (size_t)g.np0 * g.np1 * g.np2;
+  const long most = std::min<long>({16, nslots, (long)(cap_bytes / grid)});
+  long best = 1, cost = 0;
+  for (long k = 1; k <= most; ++k) {
+    const long c = (g.np2 * k + 256L * p->wgs - 1) / (256L * p->wgs) * ((nslots + k - 1) / k);
+    if (k == 1 || c < cost) {
+      best = k;
+      cost = c;
+    }
+  }
+  return (int)best;
+}
+
+int pipeline_density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
+  const PlaneOps* p = plane_ops(b, prec);
+  return p ? plane_parts(b, p, nslots, cap_bytes) : density_parts(b, nslots, prec, cap_bytes);
+}
+
+int pipeline_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* dens, double* rho) {
   const int cd = a.mode == SLOT_COMPLEX ? 1 : 0;
   // slot ranges actually used (every one non-empty)
   const int spw = (a.nslots + a.dens_parts - 1) / a.dens_parts;
   const int parts = (a.nslots + spw - 1) / spw;
   double* out = parts > 1 ? a.dens_part : rho;
-  const int r =
-      a.prec == PREC_FP64
-          ? xpass_t<double, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density")
-          : xpass_t<float, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density");
+  int r;
+  if (const PlaneOps* p = plane_ops(b, a.prec)) {
+    if (int e = bwd_z(ctx, b, a)) return e;
+    r = plane_pass(ctx, b, a, p->density, spw, nullptr, out, dens, cd, 1.0, "plane_density");
+  } else {
+    if (int e = bwd_yz(ctx, b, a)) return e;
+    r = a.prec == PREC_FP64
+            ? xpass_t<double, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density")
+            : xpass_t<float, X_DENSITY>(ctx, b, a, nullptr, out, dens, 1.0, cd, "xpass_density");
+  }
   if (r || parts == 1) return r;
   const long N = (long)b->g.np0 * b->g.np1 * b->g.np2;
   TimedLaunch tl(ctx, "density_sum");
@@ -294,7 +348,7 @@ int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* 
       p.psi = d ? bs[d - 1] : a;
       p.ld = d ? ldb : lda;
       p.t2 = const_cast<cplx<double>*>(f.t2[d]);
-      if (int e = pipeline_bwd_yz(ctx, b, p)) return e;
+      if (int e = bwd_yz(ctx, b, p)) return e;
     }
     const int pn = std::min(parts, p.nslots);
     const int spw = (p.nslots + pn - 1) / pn, used = (p.nslots + spw - 1) / spw;

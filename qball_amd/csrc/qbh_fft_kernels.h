@@ -1356,6 +1356,17 @@ k_density_sum(long N, int nparts, double scale, const double* __restrict__ part,
 }
 
 // ------------------------------------------------------------------------------------
+// y and x passes in one kernel (FP64, both edges n; qbh_fft_plane.h)
+struct PlaneOps {
+  using Launch = void (*)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
+                          const double* in, double* out, const double* dens, int cplx_density,
+                          double scale);
+  bool (*fits)(const GridDev& g) = nullptr;
+  int wgs = 0;  // workgroups per compute unit
+  Launch vmul = nullptr, density = nullptr;
+  Launch store = nullptr, load = nullptr, load_real = nullptr;  // null: separate passes
+};
+
 // Launches.  EdgeOps holds the launch functions of one edge length and precision: the
 // z, y and x passes pick theirs by the length of their own axis.
 struct EdgeOps {
@@ -1379,10 +1390,7 @@ struct EdgeOps {
   // band sums of products (FP64): nb fields b of 1 (real part) or 3 (imaginary part)
   void (*xcross)(hipStream_t st, const GridDev& g, const CrossFields& fields, int nslots, int spw,
                  int nb, const double* w, double* part);
-  // y, x and y passes of Hψ in one kernel (FP64, both edges n): its LDS for nlx lines and
-  // launch (null for the edges whose plane never fits)
-  bool (*plane_fits)(const GridDev& g);
-  void (*plane)(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw, const double* v);
+  PlaneOps plane;
 };
 
 // register-transform edges compiled by unit `part` (qbh_fft_edges.hip)
@@ -1520,8 +1528,7 @@ constexpr EdgeOps make_edge() {
                  launch_x2<T, X_DENSITY, N1, N2>,
                  launch_xload2<T, N1, N2>,
                  sizeof(T) == 8 ? launch_xcross2<N1, N2> : nullptr,
-                 PlaneOps<T, N1, N2>::fits(),
-                 PlaneOps<T, N1, N2>::launch()};
+                 plane_edge<T, N1, N2>()};
 }
 
 }  // namespace qbh

@@ -163,19 +163,18 @@ struct PipelineArgs {
   double* dens_part = nullptr;
 };
 
-int pipeline_bwd_yz(Ctx* ctx, Basis* b, const PipelineArgs& a);
-int pipeline_fwd_zy_accumulate(Ctx* ctx, Basis* b, const PipelineArgs& a, double* hpsi,
-                               long ldh, const double* kin /*0.5|k+G|^2 or null*/,
-                               int store /*0: hpsi += kinetic, FP32 term, value; 1: hpsi =
-                                           value; 2: hpsi = kinetic + FP32 term + value*/);
-// hpsi from psi: backward, times v, forward (store as for pipeline_fwd_zy_accumulate)
+// hpsi from psi: backward, times v, forward
 int pipeline_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v, double* hpsi,
-                  long ldh, const double* kin, int store);
-int pipeline_x_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f /*complex grid*/);
-int pipeline_x_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, int real_input,
-                    double scale);
-int pipeline_x_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* facs,
-                       double* rho);
+                  long ldh, const double* kin /*0.5|k+G|^2 or null*/,
+                  int store /*0: hpsi += kinetic, FP32 term, value; 1: hpsi = value; 2: hpsi =
+                              kinetic + FP32 term + value*/);
+// psi to the complex grids f
+int pipeline_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f);
+// grids f (complex, or real times scale) to coefficients out
+int pipeline_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, int real_input,
+                  double scale, double* out, long ldo);
+// rho += band sum of psi
+int pipeline_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* facs, double* rho);
 // Band sums of products of transforms, for the edges cross_edge() names (FP64):
 //   nb 1: out[r] += scale sum_n w_n Re(conj(a_n(r)) b_n(r))
 //   nb 3: out[d N + r] += scale sum_n w_n Im(conj(a_n(r)) b_{d,n}(r))
@@ -185,11 +184,8 @@ bool cross_edge(const Basis* b);
 int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* const* bs,
                    long ldb, int nbands, int nb, const double* w, double scale, double* out);
 size_t slot_bytes(const Basis* b, int prec);
-// Slot ranges of the density x pass for chunks of nslots slots: each workgroup sums all slots
-// of its rows, so the rows alone give np2 * np1 / rows-per-workgroup workgroups (216 at 72^3,
-// 1260 at 140^3: 2.5 rounds of two per CU).  Ranges for about 4096 workgroups, at least 4
-// slots each, with at most cap_bytes of partial grids.
-int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes);
+// Slot ranges of the density for chunks of nslots slots, with at most cap_bytes of partial grids
+int pipeline_density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes);
 // S (M x N, ld M) = alpha * A^T B - a0 b0^T over the real view with K rows (real != 0, the
 // Γ metric when alpha = 2) or A^H B (complex, K rows); K-split dgemm/zgemm (qbh_dense.hip)
 int band_product(Ctx* c, void* blas, bool real, int M, int N, long K, const double* A, long lda,

@@ -261,3 +261,65 @@ def test_plane_vmul(gpu_ctx, n, np2, ecut, nb, real):
     assert rel_err(from_dev(hd, basis.ngw, nb), ref) <= 1e-12
     ham.close()
     basis.close()
+
+
+@pytest.mark.parametrize("n,np2,ecut,nb,real", [
+    (18, 20, 12.0, 1, True), (28, 18, 25.0, 3, False), (40, 30, 25.0, 7, True),
+    (48, 50, 170.0, 3, True), (64, 30, 60.0, 66, False), (72, 36, 60.0, 37, True),
+    (80, 20, 25.0, 4, False), (90, 20, 25.0, 3, True), (100, 28, 60.0, 2, False)])
+def test_plane_grids(gpu_ctx, n, np2, ecut, nb, real):
+    """Grid transforms and density on square cross-sections (y and x pass in one kernel): one
+    and several slots per workgroup and slot ranges, added to what the density grid holds."""
+    import torch
+    from oracle import fft as offt
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=ecut, nbands=nb, seed=43, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), n, n, np2)
+    r, c = sysm.rods, sysm.psi
+    basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"],
+                  (n, n, np2), sysm.b)
+    N, cd = basis.N, to_dev(c)
+    rng = np.random.default_rng(n)
+    nslots = (nb + 1) // 2 if real else nb
+    f = torch.zeros(2 * nslots * N, dtype=torch.float64, device="cuda")
+    g = rng.standard_normal((nslots, N)) + 1j * rng.standard_normal((nslots, N))
+    gd = torch.from_numpy(g.view(np.float64).ravel().copy()).cuda()
+    h = rng.standard_normal(N)
+    hd, rho0 = real_to_dev(h), rng.standard_normal(N)
+    rho = real_to_dev(rho0)
+    back, one = torch.zeros_like(cd), torch.zeros(2 * basis.ngw, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    gpu_ctx.timing_report()
+    gpu_ctx.set_timing(True)
+    basis.backward(cd.data_ptr(), basis.ngw, nb, real, f.data_ptr())
+    basis.forward(gd.data_ptr(), nb, real, back.data_ptr(), basis.ngw)
+    basis.forward_real(hd.data_ptr(), 0.7, one.data_ptr())
+    basis.density(cd.data_ptr(), basis.ngw, nb, sysm.occ, 1.0, sysm.omega, rho.data_ptr())
+    gpu_ctx.sync()
+    ran = gpu_ctx.timing_report()
+    gpu_ctx.set_timing(False)
+    assert "plane_density" in ran
+    assert ({"plane_store", "plane_load"} <= set(ran)) == (n <= 64)
+    fg = f.cpu().numpy().view(np.complex128).reshape(nslots, N)
+    bg = from_dev(back, basis.ngw, nb)
+    shape = (np2, n, n)
+    for s in range(nslots):
+        if real:
+            two = 2 * s + 1 < nb
+            ref = offt.backward(maps, c[:, 2 * s], c[:, 2 * s + 1] if two else None)
+            c1, c2 = offt.forward(maps, g[s].reshape(shape), pair=True)
+            assert rel_err(bg[:, 2 * s], c1) <= 1e-12
+            if two:
+                assert rel_err(bg[:, 2 * s + 1], c2) <= 1e-12
+        else:
+            ref = offt.backward(maps, c[:, s])
+            assert rel_err(bg[:, s], offt.forward(maps, g[s].reshape(shape))) <= 1e-12
+        assert rel_err(fg[s], ref.ravel()) <= 1e-12
+    assert rel_err(from_dev(one, basis.ngw, 1)[:, 0],
+                   offt.forward(maps, 0.7 * h.reshape(shape))) <= 1e-12
+    ref = rho0 + oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)
+    assert rel_err(rho.cpu().numpy(), ref) <= 1e-12
+    basis.close()
