@@ -583,7 +583,11 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
     dfac = static_cast<double*>(aux_get(c, nfac * sizeof(double)));
   }
   if (!dfac) return fail(c, QBH_ERR_ALLOC, "density factor allocation failed");
-  hipMemcpyAsync(dfac, fac.data(), nst * sizeof(double), hipMemcpyHostToDevice, c->stream);
+  // (from the pinned block the copy does not wait; the call's synchronisation frees it)
+  const double* hfac = fac.data();
+  if (nst <= PIN_SIZE - PIN_FACS)
+    hfac = std::copy(fac.begin(), fac.end(), c->pin + PIN_FACS) - nst;
+  hipMemcpyAsync(dfac, hfac, nst * sizeof(double), hipMemcpyHostToDevice, c->stream);
   double* slotf = dfac + nst;
   int r = for_chunks(c, b, nslots, prec, [&](PipelineArgs& a, int s0) {
     a.psi = psi_dev;

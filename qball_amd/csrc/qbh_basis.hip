@@ -61,6 +61,19 @@ void* aux_get(Ctx* ctx, size_t bytes) {
   return grow_workspace(ctx, ctx->aux, ctx->aux_bytes, bytes);
 }
 
+CallBuffer::CallBuffer(Ctx* c, size_t bytes) {
+  if (bytes <= size_t(256) << 20) {
+    p = grow_workspace(c, c->call, c->call_bytes, bytes);
+  } else if (hipMalloc(&p, bytes) == hipSuccess) {
+    own = true;
+  } else {
+    p = nullptr;
+  }
+}
+CallBuffer::~CallBuffer() {
+  if (own) hipFree(p);
+}
+
 }  // namespace qbh
 
 static int set_err(Ctx* c, int code, const std::string& msg) {
@@ -86,6 +99,11 @@ extern "C" int qbh_ctx_create(int device, void* stream, qbh_ctx* out) {
       return QBH_ERR_DEVICE;
     }
     h->c.own_stream = true;
+  }
+  if (hipHostMalloc(reinterpret_cast<void**>(&h->c.pin), PIN_SIZE * sizeof(double)) != hipSuccess) {
+    if (h->c.own_stream) hipStreamDestroy(h->c.stream);
+    delete h;
+    return QBH_ERR_ALLOC;
   }
   qbh::noalloc_scratch_setup(&h->c);
   *out = h;
@@ -113,6 +131,8 @@ extern "C" int qbh_ctx_destroy(qbh_ctx ctx) {
   if (ctx->c.ev_join) hipEventDestroy(ctx->c.ev_join);
   if (ctx->c.ws) hipFree(ctx->c.ws);
   if (ctx->c.aux) hipFree(ctx->c.aux);
+  if (ctx->c.call) hipFree(ctx->c.call);
+  if (ctx->c.pin) hipHostFree(ctx->c.pin);
   if (ctx->c.own_stream) hipStreamDestroy(ctx->c.stream);
   delete ctx;
   return QBH_OK;

@@ -109,6 +109,12 @@ struct Ctx {
   // second workspace, for what a call needs beside the transform workspace
   void* aux = nullptr;
   size_t aux_bytes = 0;
+  // third one: buffers of a whole call (CallBuffer)
+  void* call = nullptr;
+  size_t call_bytes = 0;
+  // pinned host block for the scalars that kernels return (PIN_* offsets): a kernel stores them
+  // there and the call reads them after its stream synchronisation, without a copy
+  double* pin = nullptr;
   // autotuner results per problem shape (key -> knob values)
   std::map<std::string, std::vector<int>> tune_cache;
   // this device's allocation-free transform scratch (device address of the file-scope
@@ -120,6 +126,23 @@ struct Ctx {
 // Looks up (once per device, with `device` current) the device address of the
 // allocation-free scratch array and stores it in c->scratch (qbh_api.hip).
 void noalloc_scratch_setup(Ctx* c);
+
+enum { PIN_ENL = 0, PIN_PSDA = 1, PIN_EKIN = 3, PIN_VHXC = 4, PIN_FACS = 16, PIN_SIZE = 4096 };
+
+// Device memory for the length of one call that ends with a stream synchronisation: up to 256
+// MiB of the context's own, kept until it is destroyed; more is allocated and freed.  With the
+// scalars in the pinned block instead of copied back (MI355X): two SCF cycles of 108 Al atoms
+// 24.9 -> 23.7 ms, ETRS steps of 64 Si atoms 9.1 -> 8.6 ms, one Hψ of them 305 -> 298 us.
+struct CallBuffer {
+  void* p = nullptr;
+  CallBuffer(Ctx* c, size_t bytes);
+  ~CallBuffer();
+  CallBuffer(const CallBuffer&) = delete;
+  CallBuffer& operator=(const CallBuffer&) = delete;
+
+ private:
+  bool own = false;
+};
 
 // Records the named kernel's launch window when timing is enabled.
 struct TimedLaunch {

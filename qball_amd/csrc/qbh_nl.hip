@@ -303,7 +303,8 @@ k_fnl_finish_cplx(int P, int nst, T* __restrict__ F, int nsplit, long pstride,
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-__global__ void k_sum_partials(int n, double* __restrict__ partial) {
+__global__ void k_sum_partials(int n, const double* __restrict__ partial,
+                               double* __restrict__ out) {
   __shared__ double red[256];
   double e = 0.0;
   for (int i = threadIdx.x; i < n; i += 256) e += partial[i];
@@ -313,7 +314,7 @@ __global__ void k_sum_partials(int n, double* __restrict__ partial) {
     if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) partial[n] = red[0];
+  if (threadIdx.x == 0) *out = red[0];
 }
 
 // psi (FP64, ld complex) -> compact FP32 copy (2*ngw floats per band)
@@ -832,7 +833,7 @@ int nl_apply(Ham* h, const double* psi, long ld, int nst, const double* occ_host
   }
   if (enl) {
     // Enl is reduced on the device; nl_read_enl fetches it once the stream has drained
-    k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red);
+    k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red, c->pin + PIN_ENL);
     *enl = 0.0;
   }
   return 0;
@@ -1020,7 +1021,7 @@ int nl_forces(Ham* h, const double* psi, long ld, int nst, const double* occ_hos
                            static_cast<const float*>(fs.F), occ, dpsi, g);
   }
   if (r) return r;
-  if (enl) k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red);
+  if (enl) k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red, c->pin + PIN_ENL);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     c->last_error = std::string("nonlocal forces: ") + hipGetErrorString(err);
@@ -1028,12 +1029,12 @@ int nl_forces(Ham* h, const double* psi, long ld, int nst, const double* occ_hos
   }
   std::vector<double> gh(3 * (size_t)P);
   hipMemcpyAsync(gh.data(), g, gh.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream);
-  if (enl) hipMemcpyAsync(enl, h->red + kRedBlocks, sizeof(double), hipMemcpyDeviceToHost, c->stream);
   err = hipStreamSynchronize(c->stream);
   if (err != hipSuccess) {
     c->last_error = std::string("nonlocal forces: ") + hipGetErrorString(err);
     return QBH_ERR_DEVICE;
   }
+  if (enl) *enl = c->pin[PIN_ENL];
   // tmpfion[3*ia+j] -= ... summed over the columns of each atom (:2283-2288)
   for (int j = 0; j < 3; ++j)
     for (int p = 0; p < P; ++p) fion[3L * h->col_atom_host[p] + j] -= gh[(size_t)j * P + p];
@@ -1061,11 +1062,9 @@ extern "C" int qbh_ctx_library_info(qbh_ctx ctx, char* buf, int cap) {
 namespace qbh {
 
 double nl_read_enl(Ham* h, hipStream_t s) {
-  double v = 0.0;
   if (!h->red || h->P == 0) return 0.0;
-  hipMemcpyAsync(&v, h->red + kRedBlocks, sizeof(double), hipMemcpyDeviceToHost, s);
   hipStreamSynchronize(s);
-  return v;
+  return h->ctx->pin[PIN_ENL];
 }
 
 }  // namespace qbh

@@ -104,9 +104,9 @@ extern "C" int qbh_current(qbh_basis basis, const double* psi_dev, long ld, int 
   }
   const size_t bytes = sizeof(double) * ((fused ? 0 : 2 * 4 * (size_t)nb * N) + 2 * 3 * (size_t)nb * ngw +
                                          (j_dev ? 0 : 3 * (size_t)N) + nst + 3 * nblk);
-  double* buf = nullptr;
-  if (hipMalloc(&buf, bytes) != hipSuccess)
-    return ofail(c, QBH_ERR_ALLOC, "current scratch allocation failed");
+  CallBuffer hold(c, bytes);
+  double* buf = static_cast<double*>(hold.p);
+  if (!buf) return ofail(c, QBH_ERR_ALLOC, "current scratch allocation failed");
   double* f0 = buf;
   double* fd = f0 + 2 * (size_t)nb * N;
   double* ikc = fused ? buf : fd + 2 * 3 * (size_t)nb * N;
@@ -143,7 +143,6 @@ extern "C" int qbh_current(qbh_basis basis, const double* psi_dev, long ld, int 
     hipMemcpyAsync(hp.data(), part, 3 * nblk * sizeof(double), hipMemcpyDeviceToHost, c->stream);
   }
   hipStreamSynchronize(c->stream);
-  hipFree(buf);
   if (r) return r;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ofail(c, QBH_ERR_DEVICE, std::string("current: ") + hipGetErrorString(e));

@@ -390,12 +390,9 @@ extern "C" int qbh_psda_update(qbh_psda p, double* psi_dev, long ld, double* hps
   } else {
     k_precondition<true><<<grid, 256, 0, c->stream>>>(ngw, nst, real ? 1 : 0, p->K, p->occ,
                                                       hpsi_dev, ldh, p->dcl, p->part);
-    double* sums = p->part + 2 * kPart;
-    k_sum_parts<<<2, 256, 0, c->stream>>>(grid.x * grid.y, p->part, sums);
-    double hp[2] = {0.0, 0.0};
-    hipMemcpyAsync(hp, sums, sizeof(hp), hipMemcpyDeviceToHost, c->stream);
+    k_sum_parts<<<2, 256, 0, c->stream>>>(grid.x * grid.y, p->part, c->pin + PIN_PSDA);
     hipStreamSynchronize(c->stream);
-    const double a = hp[0], b = hp[1];
+    const double a = c->pin[PIN_PSDA], b = c->pin[PIN_PSDA + 1];
     if (b != 0.0) th = -a / b;
     if (th < -1.0) th = 0.0;
     th = std::min(2.0, th);
@@ -420,9 +417,9 @@ extern "C" int qbh_kinetic_energy(qbh_basis basis, const double* psi_dev, long l
   double* part = d + nst;
   k_ekin<<<grid, 256, 0, c->stream>>>(b->g.ngw, nst, b->g.real ? 1 : 0, b->kpg2, d, psi_dev, ld,
                                       part);
-  k_sum_parts<<<1, 256, 0, c->stream>>>(grid.x * grid.y, part, part + kPart);
-  hipMemcpyAsync(ekin, part + kPart, sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  k_sum_parts<<<1, 256, 0, c->stream>>>(grid.x * grid.y, part, c->pin + PIN_EKIN);
   hipStreamSynchronize(c->stream);
+  *ekin = c->pin[PIN_EKIN];
   return scheck(c, "kinetic energy");
 }
 

@@ -125,6 +125,22 @@ __global__ void k_add_real_part(long n, const double* __restrict__ f, double* __
   if (i < n) vr[i] += f[2 * i];
 }
 
+// out[k] = sum of the n partials of quantity k = blockIdx.x < 3; out[3..4], out[5..6] = vion
+// (0 without) and rho at G = 0
+__global__ void __launch_bounds__(256)
+k_vhxc_sums(int n, const double* __restrict__ part, const double* __restrict__ vion,
+            const double* __restrict__ rho, double* __restrict__ out) {
+  __shared__ double red[256];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[(long)blockIdx.x * n + i];
+  s = block_sum(s, red);
+  if (threadIdx.x == 0) out[blockIdx.x] = s;
+  if (blockIdx.x == 0 && threadIdx.x < 2) {
+    out[3 + threadIdx.x] = vion ? vion[threadIdx.x] : 0.0;
+    out[5 + threadIdx.x] = rho[threadIdx.x];
+  }
+}
+
 static int vfail(Ctx* c, int code, const std::string& m) {
   c->last_error = m;
   return code;
@@ -142,14 +158,11 @@ extern "C" int qbh_update_vhxc(qbh_basis vbasis, const double* rhor_dev, const d
   const long N = (long)g.np0 * g.np1 * g.np2;
   const int ngw = g.ngw;
   const int nb = 256;
-  double *part = nullptr, *vg = nullptr, *f = nullptr;
-  if (hipMalloc(&part, 3 * nb * sizeof(double)) != hipSuccess ||
-      hipMalloc(&vg, 2 * sizeof(double) * ngw) != hipSuccess ||
-      hipMalloc(&f, 2 * sizeof(double) * N) != hipSuccess) {
-    for (void* p : {(void*)part, (void*)vg, (void*)f})
-      if (p) hipFree(p);
-    return vfail(c, QBH_ERR_ALLOC, "update_vhxc scratch allocation failed");
-  }
+  CallBuffer buf(c, sizeof(double) * (3 * nb + 2 * (size_t)ngw + 2 * (size_t)N));
+  if (!buf.p) return vfail(c, QBH_ERR_ALLOC, "update_vhxc scratch allocation failed");
+  double* part = static_cast<double*>(buf.p);
+  double* f = part + 3 * nb;
+  double* vg = f + 2 * (size_t)N;
   {
     TimedLaunch tl(c, "vhxc_lda");
     k_lda<<<nb, 256, 0, c->stream>>>(N, rhor_dev, v_r_dev, part);
@@ -164,30 +177,19 @@ extern "C" int qbh_update_vhxc(qbh_basis vbasis, const double* rhor_dev, const d
     TimedLaunch tl(c, "vhxc_add");
     k_add_real_part<<<(unsigned)((N + 255) / 256), 256, 0, c->stream>>>(N, f, v_r_dev);
   }
-  std::vector<double> hp(3 * nb, 0.0);
-  hipMemcpyAsync(hp.data(), part, 3 * nb * sizeof(double), hipMemcpyDeviceToHost, c->stream);
+  double* e = c->pin + PIN_VHXC;  // exc, eps, eh; vion and rho at G = 0
+  k_vhxc_sums<<<3, 256, 0, c->stream>>>(nb, part, vion_g_dev, rhog_dev, e);
   hipStreamSynchronize(c->stream);
-  for (void* p : {(void*)part, (void*)vg, (void*)f}) hipFree(p);
   if (r) return r;
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return vfail(c, QBH_ERR_DEVICE, hipGetErrorString(e));
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return vfail(c, QBH_ERR_DEVICE, hipGetErrorString(err));
   if (energies) {
-    double exc = 0.0, eps = 0.0, eh = 0.0;
-    for (int i = 0; i < nb; ++i) {
-      exc += hp[i];
-      eps += hp[nb + i];
-      eh += hp[2 * nb + i];
-    }
+    double eps = e[1];
     // Γ half-sphere sums count G and -G: 2 * sum - G=0 term (EnergyFunctional.cc:463-467)
-    if (g.real) {
-      std::vector<double> v0(2, 0.0), r0(2, 0.0);
-      if (vion_g_dev) hipMemcpy(v0.data(), vion_g_dev, 2 * sizeof(double), hipMemcpyDeviceToHost);
-      hipMemcpy(r0.data(), rhog_dev, 2 * sizeof(double), hipMemcpyDeviceToHost);
-      eps = 2.0 * eps - (r0[0] / omega * v0[0] + r0[1] / omega * v0[1]);
-    }
+    if (g.real) eps = 2.0 * eps - (e[5] / omega * e[3] + e[6] / omega * e[4]);
     energies[0] = eps * omega;                                   // eps
-    energies[1] = (g.real ? 1.0 : 0.5) * omega * 4.0 * M_PI * eh;  // ehart
-    energies[2] = exc * omega / (double)N;                       // exc
+    energies[1] = (g.real ? 1.0 : 0.5) * omega * 4.0 * M_PI * e[2];  // ehart
+    energies[2] = e[0] * omega / (double)N;                       // exc
   }
   return QBH_OK;
 }
