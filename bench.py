@@ -102,6 +102,7 @@ def kernel_bytes(sysm, nslots, prec_bytes):
         "xpass_vmul": nslots * (2 * t2) + N * 8,
         "ypass_fwd": nslots * (t2 + t1),
         "zpass_fwd": nslots * (t1 + psi_pair + 2 * psi_pair),
+        "plane_vmul": nslots * (2 * t1) + N * 8,  # y, x and y passes of short edges in one
     }
 
 
@@ -242,7 +243,8 @@ def main():
     # the unfused pruned-pencil model of qball's FourierTransform (per Γ pair:
     # 2(2 nvec np2 s) z + 2(4 ntrans0 np0 np2 s) pruned x + 2(2 N s) y + 2(nvec np2 + N) s
     # zvec<->grid + (2 N s + N r) xv + 6 ngw s coefficients in / Hψ RMW)
-    fft_names = ("zpass_bwd", "ypass_bwd", "xpass_vmul", "ypass_fwd", "zpass_fwd")
+    fft_names = [k for k in ("zpass_bwd", "ypass_bwd", "xpass_vmul", "ypass_fwd", "zpass_fwd",
+                             "plane_vmul") if k in per_kernel]
     t_fft = sum(per_kernel[k]["avg_ms"] * per_kernel[k]["launches_per_step"] for k in fft_names)
     b_fft = sum(per_kernel[k]["bytes_per_launch"] * per_kernel[k]["launches_per_step"]
                 for k in fft_names)
