@@ -1034,7 +1034,7 @@ k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 // ------------------------------------------------------------------------------------
 // x pass of band sums of products of transforms, without a grid per band:
 //   part[range][d][r] = sum_s w_s Re (IM: Im) (conj(a_s(r)) b_{d,s}(r)),  d < NB
-// over a range of slots per blockIdx.y (w null: 1).  a and the b_d are y-transformed lines
+// over the slots with w_s > 0 of a range per blockIdx.y (w null: 1).  a and the b_d are y-transformed lines
 // (T2); a workgroup takes the NB + 1 fields of a slot one after the other through the same
 // row buffers, the next field's lines in flight, holds a(r) in registers and accumulates in
 // FP64.  Against storing the transforms as grids and multiplying them from memory (16 bytes a
@@ -1146,17 +1146,25 @@ k_xcross2(GridDev g, CrossFields fields, int nslots, int slots_per_wg,
   for (int d = 0; d < NB; ++d)
 #pragma unroll
     for (int k2 = 0; k2 < N2; ++k2) acc[d][k2] = 0.0;
-  if (s0 < s1) prefetch(fields.t2[0], s0);
+  // slots without a positive weight are left out, whatever their transforms hold (0 * NaN)
+  auto weighted = [&](int s) {
+    if (w)
+      while (s < s1 && !(w[s] > 0.0)) ++s;
+    return s;
+  };
+  int s = weighted(s0);
+  if (s < s1) prefetch(fields.t2[0], s);
   __syncthreads();
-  for (int s = s0; s < s1; ++s) {
+  while (s < s1) {
     C a[N2], b[N2];
     transform(fields.t2[1], s, a);
     const double ws = w ? w[s] : 1.0;
+    const int sn = weighted(s + 1);
 #pragma unroll
     for (int d = 0; d < NB; ++d) {
       const bool last = d + 1 == NB;
-      transform(last ? (s + 1 < s1 ? fields.t2[0] : nullptr) : fields.t2[d + 2 < 4 ? d + 2 : 0],
-                last ? s + 1 : s, b);
+      transform(last ? (sn < s1 ? fields.t2[0] : nullptr) : fields.t2[d + 2 < 4 ? d + 2 : 0],
+                last ? sn : s, b);
       if (lane < TB) {
 #pragma unroll
         for (int k2 = 0; k2 < N2; ++k2)
@@ -1164,6 +1172,7 @@ k_xcross2(GridDev g, CrossFields fields, int nslots, int slots_per_wg,
                                  : a[k2].x * b[k2].x + a[k2].y * b[k2].y);
       }
     }
+    s = sn;
   }
   if (lane < TB && rb < nyl) {
     const long N = (long)n * np1 * np2;

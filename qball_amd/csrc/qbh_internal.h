@@ -202,7 +202,7 @@ int pipeline_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* fa
 //   nb 1: out[r] += scale sum_n w_n Re(conj(a_n(r)) b_n(r))
 //   nb 3: out[d N + r] += scale sum_n w_n Im(conj(a_n(r)) b_{d,n}(r))
 // a and the nb fields b are nbands coefficient columns each (leading dimensions lda, ldb), w
-// (device, nullable = 1) one weight per band
+// (device, nullable = 1) one weight per band; bands without a positive weight are left out
 bool cross_edge(const Basis* b);
 int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* const* bs,
                    long ldb, int nbands, int nb, const double* w, double scale, double* out);

@@ -323,3 +323,35 @@ def test_plane_grids(gpu_ctx, n, np2, ecut, nb, real):
     ref = rho0 + oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)
     assert rel_err(rho.cpu().numpy(), ref) <= 1e-12
     basis.close()
+
+
+@pytest.mark.parametrize("real", (True, False))
+@pytest.mark.parametrize("grid", [(24, 36, 30), (72, 20, 36), (140, 24, 18), (22, 24, 18)])
+@pytest.mark.parametrize("occ", [(0, 2, 2, 0, 0, 1, 2, 0), (2, 0, 0, 0, 0, 0, 0, 0),
+                                 (0, 0, 0, 0, 0, 0, 0, 1), (0, 0, 0, 0, 0, 0, 0, 0)])
+def test_current_leaves_out_empty_bands(gpu_ctx, real, grid, occ):
+    """Bands without a positive weight do not enter the current, whatever they hold: NaN and
+    infinities in them leave its bits as they are with zeros there.  Grids with and without a
+    register x transform."""
+    import torch
+    from qball_amd import Basis
+    from qball_amd.workload import make_system
+    nb, occ = len(occ), np.array(occ, dtype=np.float64)
+    sysm = make_system(ncell=1, ecut_ry=25.0, nbands=nb, seed=28, complex_basis=not real)
+    r = sysm.rods
+    basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+    out = []
+    for fill in (0.0, np.nan, np.inf):
+        c = sysm.psi.copy()
+        c[:, occ == 0.0] = fill
+        cd = to_dev(c)
+        j = torch.full((3, basis.N), np.nan, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        total = basis.current(cd.data_ptr(), basis.ngw, nb, occ, 1.0, sysm.omega,
+                              j_ptr=j.data_ptr())
+        gpu_ctx.sync()
+        out.append((j.cpu().numpy(), np.array(total)))
+    assert np.isfinite(out[0][0]).all() and (real or occ.any() == out[0][0].any())
+    for j, total in out[1:]:
+        assert np.array_equal(j, out[0][0]) and np.array_equal(total, out[0][1])
+    basis.close()
