@@ -193,11 +193,11 @@ __device__ __forceinline__ void stage_b(cplx<T>* b, const cplx<T>* tw, int k1) {
   sdft<N2, DIR>(b);
 }
 
-// a[k] *= W_n^{DIR e k}, k < K, n the length of the table tw (e (K - 1) < n).  FP64 reads every
-// power from the table: local Hψ is 1.2 to 1.9 times closer to 64-bit reference transforms
-// than with the repeated products of w = tw[e] that FP32 forms (140^3: 5.3e-16 against 8.2e-16
-// of the result), in the same time (140^3 x pass, 300 slots, 3.75 against 3.73 ms).
-template <int K, int DIR, typename T>
+// a[k] *= W_n^{DIR e k}, k < K, n the length of the table tw (e (K - 1) < n).  FP64 and TAB read
+// every power from the table: local Hψ is 1.2 to 1.9 times closer to 64-bit reference transforms
+// than with the repeated products of w = tw[e] that FP32 forms otherwise (140^3: 5.3e-16 against
+// 8.2e-16 of the result), in the same time (140^3 x pass, 300 slots, 3.75 against 3.73 ms).
+template <int K, int DIR, bool TAB = false, typename T>
 __device__ __forceinline__ void twiddle_row(cplx<T>* a, const cplx<T>* tw, int e) {
   if (e == 0) return;
   cplx<T> w = tw[e];
@@ -207,7 +207,7 @@ __device__ __forceinline__ void twiddle_row(cplx<T>* a, const cplx<T>* tw, int e
   for (int k = 1; k < K; ++k) {
     a[k] = cmul(a[k], p);
     if (k + 1 < K) {
-      if constexpr (sizeof(T) == 8) {
+      if constexpr (sizeof(T) == 8 || TAB) {
         p = tw[e * (k + 1)];
         if (DIR < 0) p.y = -p.y;
       } else {
@@ -239,7 +239,8 @@ template <int N1, int N2, int ON = QBH_LDS_PAD> struct Pad {
 //   stage B: task (r, k1): DFT_N2 over the contiguous block N2*k1 + j2 -> X[k1 + N1*k2],
 //            held in registers until every lane has read its block, then stored at the
 //            natural positions.
-template <int N1, int N2, int RPW, int DIR, int PAD = QBH_LDS_PAD, typename T>
+// TAB: FP32 stage twiddles from the table too (twiddle_row).
+template <int N1, int N2, int RPW, int DIR, int PAD = QBH_LDS_PAD, bool TAB = false, typename T>
 __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const cplx<T>* tw,
                                          int lane) {
   constexpr int TA = RPW * N2, TB = RPW * N1;
@@ -255,7 +256,7 @@ __device__ __forceinline__ void rows_fft(cplx<T>* buf, int nrows, int ld, const 
 #pragma unroll
       for (int j1 = 0; j1 < N1; ++j1) a[j1] = row[S * j1];
       stage_a<N1, N2, DIR>(a, tw);
-      if constexpr (!stockham_order<T, N1, N2>()) twiddle_row<N1, DIR>(a, tw, j2);
+      if constexpr (!stockham_order<T, N1, N2>()) twiddle_row<N1, DIR, TAB>(a, tw, j2);
 #pragma unroll
       for (int k1 = 0; k1 < N1; ++k1) row[S * k1] = a[k1];
     }

@@ -963,6 +963,9 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 // stores the nlx sphere lines, YB consecutive rows of a line at a time.  Bound by HBM: it
 // reads the grid and writes T2.  With the LDS Stockham pass it replaces at these edges (198 us
 // of it) a backward and a forward transform of 65 orbitals at 72^3 took 343 us, now 208 us.
+// FP32 reads its stage twiddles from the table like the Stockham pass: with the repeated products
+// of the other FP32 passes a forward transform was 5 to 24 % further from the 64-bit one at the E
+// edges (64 along x: 1.54e-7 of the result; tabled 1.30e-7, Stockham 1.30e-7).
 template <typename T, bool REAL, int N1, int N2, int GPW>
 __global__ void __launch_bounds__(NTHR)
 k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
@@ -1021,7 +1024,7 @@ k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
       }
     }
     wave_sync();
-    rows_fft<N1, N2, LPW, -1, QBH_XLDS_PAD>(buf, nyl, LD, tw, lane);
+    rows_fft<N1, N2, LPW, -1, QBH_XLDS_PAD, true>(buf, nyl, LD, tw, lane);
     __syncthreads();
     cplx<T>* dst = t2 + s * sstride;
 #pragma unroll
@@ -1487,18 +1490,28 @@ void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
                                                          cplx_density);
 }
 
+// factors of n = n1 * n2 in the order of k_xload2: FP32 takes the one with more powers of two
+// first, like the Stockham plans, which lead with them (error of an FP32 forward transform, 72 along
+// x: 1.29e-7 of the result as 8 * 9, 1.36e-7 as 9 * 8, 1.32e-7 with the Stockham x pass)
+constexpr int twos(int n) { return n % 2 ? 0 : 1 + twos(n / 2); }
+template <typename T, int N1, int N2> struct LoadFactors {
+  static constexpr bool swap = sizeof(T) == 4 && !stockham_order<T, N1, N2>() && twos(N2) > twos(N1);
+  static constexpr int A = swap ? N2 : N1, B = swap ? N1 : N2;
+};
+
 template <typename T, int N1, int N2>
 void launch_xload2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
                    const double* f, bool real_input, double scale) {
   constexpr int n = N1 * N2, YB = x_rows(N1, N2) * NWAVE;
+  constexpr int A = LoadFactors<T, N1, N2>::A, B = LoadFactors<T, N1, N2>::B;
   constexpr int GF = (YB * n + NTHR - 1) / NTHR;
   const dim3 grid(g.np2 * ((g.np1 + YB - 1) / YB), (a.nslots + spw - 1) / spw);
-  const size_t lds = sizeof(cplx<T>) * ((size_t)n + (size_t)YB * Pad<N1, N2, QBH_XLDS_PAD>::row(n));
+  const size_t lds = sizeof(cplx<T>) * ((size_t)n + (size_t)YB * Pad<A, B, QBH_XLDS_PAD>::row(n));
   auto* t2 = static_cast<cplx<T>*>(a.t2);
   if (real_input)
-    k_xload2<T, true, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
+    k_xload2<T, true, A, B, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
   else
-    k_xload2<T, false, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
+    k_xload2<T, false, A, B, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, f, scale);
 }
 
 template <int N1, int N2>

@@ -355,3 +355,45 @@ def test_current_leaves_out_empty_bands(gpu_ctx, real, grid, occ):
     for j, total in out[1:]:
         assert np.array_equal(j, out[0][0]) and np.array_equal(total, out[0][1])
     basis.close()
+
+
+@pytest.mark.parametrize("n", (28, 32, 36, 40, 48, 50, 54, 60, 64, 72, 80, 90, 96, 100, 108, 120,
+                               128, 140, 144, 160, 168, 180, 192, 210, 224, 240, 256))
+def test_fp32_forward_error(gpu_ctx, n):
+    """FP32 forward transforms from complex and real grids are as close to the 64-bit ones with
+    the register x pass as with the Stockham one.  Both read tabled twiddles, so their errors
+    have the same size, found here from at least 8 x 1151 coefficients to about 0.7 %; the bar
+    is 2 %."""
+    import torch
+    from oracle import fft as offt
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=25.0, nbands=1, seed=23, generate_psi=False)
+    grid, shape, m = (n, 22, 22), (22, 22, n), 8
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut), *grid)
+    r = sysm.rods
+    basis = Basis(gpu_ctx, True, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+    ham = Hamiltonian(gpu_ctx, basis)  # (holds the basis' tuning)
+    rng = np.random.default_rng(n)
+    g = rng.standard_normal((m, basis.N)) + 1j * rng.standard_normal((m, basis.N))
+    rho = rng.standard_normal((2 * m, basis.N))
+    ref = [offt.forward(maps, x.reshape(shape)).ravel() for x in g]
+    ref_real = [offt.forward(maps, x.astype(np.complex128).reshape(shape)).ravel() for x in rho]
+    gd, rd = real_to_dev(g.view(np.float64).ravel()), real_to_dev(rho.ravel())
+    err = {}
+    for reg in (1, 0):
+        ham.set_tuning("x_reg", reg)
+        out = torch.zeros((m, 2 * basis.ngw), dtype=torch.float64, device="cuda")
+        real = torch.zeros((2 * m, 2 * basis.ngw), dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        basis.forward(gd.data_ptr(), m, False, out.data_ptr(), basis.ngw, 0x10)
+        for k in range(2 * m):
+            basis.forward_real(rd[k * basis.N:].data_ptr(), 1.0, real[k].data_ptr(), 0x10)
+        gpu_ctx.sync()
+        err[reg] = (rel_err(out.cpu().numpy().view(np.complex128), ref),
+                    rel_err(real.cpu().numpy().view(np.complex128), ref_real))
+    for k in range(2):
+        assert err[1][k] <= 1.02 * err[0][k], err
+    ham.close()
+    basis.close()
