@@ -504,8 +504,7 @@ int qbh::hpsi_impl(Ham* h, const double* psi, long ld, int nst, const double* oc
                                                                   hpsi, ldh);
   }
   if (int r = dev_check(c, "hpsi")) return r;
-  if (enl && do_nl) *enl = nl_read_enl(h, main);
-  return 0;
+  return enl && do_nl ? nl_read_enl(h, main, enl) : 0;
 }
 
 extern "C" int qbh_hpsi(qbh_ham ham, const double* psi_dev, long ld, int nst, const double* occ,

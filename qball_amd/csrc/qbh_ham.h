@@ -92,7 +92,8 @@ int expo_impl(Ham* h, const double* in, long ldin, double* outp, long ldout, int
 int nl_apply(Ham* h, const double* psi, long ld, int nst, const double* occ, double* hpsi,
              long ldh, int fp32, double* enl, const float** defer_add32 = nullptr,
              bool overwrite = false);
-double nl_read_enl(Ham* h, hipStream_t s);
+// Enl of the last nl_apply with enl, once stream s has drained; an error code if that fails
+int nl_read_enl(Ham* h, hipStream_t s, double* enl);
 // non-local ionic forces of qbh_nl_forces into fion (host, 3 per atom, overwritten)
 int nl_forces(Ham* h, const double* psi, long ld, int nst, const double* occ, int fp32,
               double* fion, double* enl);

@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <array>
 #include <cstdio>
+#include <limits>
 #include <map>
 #include <string>
 #include <vector>
@@ -632,6 +633,14 @@ static int nl_occ(Ham* h, int nst, const double* occ_host, const double** occ) {
   return 0;
 }
 
+// Enl into the context's pinned slot, which every Hamiltonian of the context shares: NaN until
+// the kernel has stored it, so that no earlier call's energy can be taken for this one
+static void sum_enl(Ham* h) {
+  Ctx* c = h->ctx;
+  c->pin[PIN_ENL] = std::numeric_limits<double>::quiet_NaN();
+  k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red, c->pin + PIN_ENL);
+}
+
 // The projector coefficients of an Hψ call: F = anl^T psi over the real view (Γ) or
 // anl^H psi, finished (K-slice partials summed; Γ: G=0 term and x2), with Enl partials in
 // h->red and F scaled by wt/Omega (NonLocalPotential.cc:2040-2148).  FP32: psi is first
@@ -833,7 +842,7 @@ int nl_apply(Ham* h, const double* psi, long ld, int nst, const double* occ_host
   }
   if (enl) {
     // Enl is reduced on the device; nl_read_enl fetches it once the stream has drained
-    k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red, c->pin + PIN_ENL);
+    sum_enl(h);
     *enl = 0.0;
   }
   return 0;
@@ -1021,7 +1030,7 @@ int nl_forces(Ham* h, const double* psi, long ld, int nst, const double* occ_hos
                            static_cast<const float*>(fs.F), occ, dpsi, g);
   }
   if (r) return r;
-  if (enl) k_sum_partials<<<1, 256, 0, c->stream>>>(kRedBlocks, h->red, c->pin + PIN_ENL);
+  if (enl) sum_enl(h);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     c->last_error = std::string("nonlocal forces: ") + hipGetErrorString(err);
@@ -1061,10 +1070,16 @@ extern "C" int qbh_ctx_library_info(qbh_ctx ctx, char* buf, int cap) {
 
 namespace qbh {
 
-double nl_read_enl(Ham* h, hipStream_t s) {
-  if (!h->red || h->P == 0) return 0.0;
-  hipStreamSynchronize(s);
-  return h->ctx->pin[PIN_ENL];
+int nl_read_enl(Ham* h, hipStream_t s, double* enl) {
+  *enl = 0.0;
+  if (!h->red || h->P == 0) return 0;
+  const hipError_t err = hipStreamSynchronize(s);
+  if (err != hipSuccess) {
+    h->ctx->last_error = std::string("nonlocal energy: ") + hipGetErrorString(err);
+    return QBH_ERR_DEVICE;
+  }
+  *enl = h->ctx->pin[PIN_ENL];
+  return 0;
 }
 
 }  // namespace qbh

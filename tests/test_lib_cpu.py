@@ -62,3 +62,42 @@ def test_workload_density_grid_matches_oracle():
     from qball_amd.workload import density_grid_np
     a = np.diag([20.52] * 3)
     assert density_grid_np(a, 12.5) == density_grid(UnitCell(a), 12.5)[1]
+
+
+def test_enl_of_a_failed_call_is_an_error(tmp_path):
+    """nl_read_enl on a Hamiltonian whose stream cannot be synchronised (no device here) reports
+    it instead of returning what an earlier call left in the pinned slot."""
+    import shutil
+    import subprocess
+    import torch
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if torch.cuda.is_available():
+        pytest.skip("a GPU is present")
+    from qball_amd import lib
+    lib()
+    src = tmp_path / "enl.hip"
+    src.write_text("""
+#include "qbh_ham.h"
+#include <cstdio>
+int main() {
+  double pin[qbh::PIN_SIZE] = {}, red = 0.0, enl = -1.0;
+  pin[qbh::PIN_ENL] = 42.0;  // an earlier call's energy
+  qbh::Ctx c;
+  c.pin = pin;
+  qbh::Ham h;
+  h.ctx = &c;
+  h.P = 1;
+  h.red = &red;
+  const int r = qbh::nl_read_enl(&h, nullptr, &enl);
+  c.pin = nullptr;
+  std::printf("%d %g %zu\\n", r, enl, c.last_error.size());
+}
+""")
+    pkg = os.path.join(ROOT, "qball_amd")
+    obj, exe = str(tmp_path / "enl.o"), str(tmp_path / "enl")
+    subprocess.run([hipcc, "-std=c++17", "--cuda-host-only", "-I" + os.path.join(pkg, "csrc"), "-c",
+                    str(src), "-o", obj], check=True)
+    subprocess.run([hipcc, obj, "-o", exe, "-L" + pkg, "-lqbh", "-Wl,-rpath," + pkg], check=True)
+    rc, enl, msg = subprocess.run([exe], check=True, capture_output=True,
+                                  text=True).stdout.split()
+    assert int(rc) != 0 and float(enl) != 42.0 and int(msg) > 0
