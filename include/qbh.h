@@ -51,7 +51,10 @@ int qbh_ctx_create(int device, void* stream, qbh_ctx* out);
 int qbh_ctx_destroy(qbh_ctx ctx);
 const char* qbh_last_error(qbh_ctx ctx);
 int qbh_sync(qbh_ctx ctx);
-/* Cap (bytes) on the transform workspace the library keeps per context. */
+/* Cap (bytes) on the transform workspace the library keeps per context (it holds one transform
+ * at least).  Beside it the context keeps at most two blocks for temporaries of its calls, each
+ * no larger than the cap and 256 MiB; larger temporaries are allocated and freed by the call.
+ * Blocks kept under an earlier, larger cap stay until the context is destroyed. */
 int qbh_ctx_set_workspace_cap(qbh_ctx ctx, double bytes);
 /* Per-kernel timing with HIP events on the context's stream (0 = off). */
 int qbh_ctx_set_timing(qbh_ctx ctx, int on);

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -568,19 +569,20 @@ extern "C" int qbh_density(qbh_basis basis, const double* psi_dev, long ld, int 
   const bool pair = b->g.real;
   const int nslots = pair ? (nst + 1) / 2 : nst;
   const long N = (long)b->g.np0 * b->g.np1 * b->g.np2;
-  // band and slot factors, and the partial grids of the slot ranges (at most 256 MiB and the
-  // caller's workspace cap; without memory for them, one range)
+  // band and slot factors, and the partial grids of the slot ranges (as many as the kept block
+  // takes; without memory for them, one range)
   const size_t nfac = ((nst + 4 * (size_t)nslots + 31) / 32) * 32;
   const size_t chunk = std::max<size_t>(1, c->ws_cap / slot_bytes(b, prec));
+  const size_t fbytes = nfac * sizeof(double), room = kept_cap(c);
   int parts = pipeline_density_parts(b, (int)std::min<size_t>(nslots, chunk), prec,
-                            std::min<size_t>(c->ws_cap, size_t(256) << 20));
-  double* dfac = nullptr;
-  if (parts > 1)
-    dfac = static_cast<double*>(aux_get(c, (nfac + (size_t)parts * N) * sizeof(double)));
-  if (!dfac) {
+                                     room > fbytes ? room - fbytes : 0);
+  std::optional<CallBuffer> buf;
+  buf.emplace(c, fbytes + (parts > 1 ? parts * N * sizeof(double) : 0));
+  if (!buf->p && parts > 1) {
     parts = 1;
-    dfac = static_cast<double*>(aux_get(c, nfac * sizeof(double)));
+    buf.emplace(c, fbytes);
   }
+  double* dfac = static_cast<double*>(buf->p);
   if (!dfac) return fail(c, QBH_ERR_ALLOC, "density factor allocation failed");
   // (from the pinned block the copy does not wait; the call's synchronisation frees it)
   const double* hfac = fac.data();

@@ -57,21 +57,26 @@ static void* grow_workspace(Ctx* ctx, void*& ws, size_t& have, size_t bytes) {
 }
 
 void* ws_get(Ctx* ctx, size_t bytes) { return grow_workspace(ctx, ctx->ws, ctx->ws_bytes, bytes); }
-void* aux_get(Ctx* ctx, size_t bytes) {
-  return grow_workspace(ctx, ctx->aux, ctx->aux_bytes, bytes);
-}
 
-CallBuffer::CallBuffer(Ctx* c, size_t bytes) {
-  if (bytes <= size_t(256) << 20) {
-    p = grow_workspace(c, c->call, c->call_bytes, bytes);
+size_t kept_cap(const Ctx* c) { return std::min<size_t>(c->ws_cap, size_t(256) << 20); }
+
+CallBuffer::CallBuffer(Ctx* c, size_t bytes, Ctx::Kept Ctx::*slot) {
+  Ctx::Kept& k = c->*slot;
+  if (bytes <= std::max(kept_cap(c), k.bytes)) {
+    p = grow_workspace(c, k.p, k.bytes, bytes);
+  } else if (t_capturing) {
+    p = nullptr;
   } else if (hipMalloc(&p, bytes) == hipSuccess) {
-    own = true;
+    own = c;
   } else {
+    (void)hipGetLastError();
     p = nullptr;
   }
 }
 CallBuffer::~CallBuffer() {
-  if (own) hipFree(p);
+  if (!own) return;
+  hipStreamSynchronize(own->stream);
+  hipFree(p);
 }
 
 }  // namespace qbh
@@ -130,8 +135,8 @@ extern "C" int qbh_ctx_destroy(qbh_ctx ctx) {
   if (ctx->c.ev_fork) hipEventDestroy(ctx->c.ev_fork);
   if (ctx->c.ev_join) hipEventDestroy(ctx->c.ev_join);
   if (ctx->c.ws) hipFree(ctx->c.ws);
-  if (ctx->c.aux) hipFree(ctx->c.aux);
-  if (ctx->c.call) hipFree(ctx->c.call);
+  for (const qbh::Ctx::Kept* k : {&ctx->c.call, &ctx->c.inner})
+    if (k->p) hipFree(k->p);
   if (ctx->c.pin) hipHostFree(ctx->c.pin);
   if (ctx->c.own_stream) hipStreamDestroy(ctx->c.stream);
   delete ctx;

@@ -355,7 +355,8 @@ static int gram_real(Ctx* c, int n, long K, double* psi, long ld, int* hinfo) {
   const int slices = mfma_sym_slices(n, K);
   const size_t nn = (size_t)n * n;
   // partials, S, W, T and the pivot flag
-  double* P = static_cast<double*>(aux_get(c, sizeof(double) * ((slices + 3) * nn + 2)));
+  CallBuffer buf(c, sizeof(double) * ((slices + 3) * nn + 2));
+  double* P = static_cast<double*>(buf.p);
   // rotated bands, whole or a range of coefficients at a time within the workspace cap
   const size_t room = std::max<size_t>(c->ws_cap / (8 * (size_t)n), 128);
   const long w = (size_t)K <= room ? K : (long)(room / 128 * 128);

@@ -1,6 +1,7 @@
 // G-sphere <-> grid transform pipeline: dispatch by edge length, and the LDS Stockham forms
 // of the passes (the kernels and their design are in qbh_fft_kernels.h).
 #include <cstdio>
+#include <optional>
 
 #include "qbh_fft_edges.h"
 #include "qbh_fft_kernels.h"
@@ -324,11 +325,11 @@ int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* 
   const int S = (int)std::min<size_t>({std::max<size_t>(1, ctx->ws_cap / per), (size_t)nbands, 65535});
   char* ws = static_cast<char*>(ws_get(ctx, S * per));
   // partial grids per slot range: one range at least, more as for the density
-  const size_t cap = std::min<size_t>(ctx->ws_cap, size_t(256) << 20) / nb;
-  int parts = density_parts(b, S, PREC_FP64, cap);
-  double* part = static_cast<double*>(aux_get(ctx, sizeof(double) * parts * nb * N));
-  if (!part && parts > 1)
-    part = static_cast<double*>(aux_get(ctx, sizeof(double) * (parts = 1) * nb * N));
+  int parts = density_parts(b, S, PREC_FP64, kept_cap(ctx) / nb);
+  std::optional<CallBuffer> buf;
+  buf.emplace(ctx, sizeof(double) * parts * nb * N, &Ctx::inner);
+  if (!buf->p && parts > 1) buf.emplace(ctx, sizeof(double) * (parts = 1) * nb * N, &Ctx::inner);
+  double* part = static_cast<double*>(buf->p);
   if (!ws || !part) {
     ctx->last_error = "transform workspace allocation failed";
     return -2;

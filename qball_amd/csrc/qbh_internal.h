@@ -106,12 +106,11 @@ struct Ctx {
   void* ws = nullptr;
   size_t ws_bytes = 0;
   size_t ws_cap = size_t(8) << 30;  // cap on pipeline workspace
-  // second workspace, for what a call needs beside the transform workspace
-  void* aux = nullptr;
-  size_t aux_bytes = 0;
-  // third one: buffers of a whole call (CallBuffer)
-  void* call = nullptr;
-  size_t call_bytes = 0;
+  // blocks kept for CallBuffer: of a whole call, and of the band sums that run inside one
+  struct Kept {
+    void* p = nullptr;
+    size_t bytes = 0;
+  } call, inner;
   // pinned host block for the scalars that kernels return (PIN_* offsets): a kernel stores them
   // there and the call reads them after its stream synchronisation, without a copy
   double* pin = nullptr;
@@ -129,20 +128,24 @@ void noalloc_scratch_setup(Ctx* c);
 
 enum { PIN_ENL = 0, PIN_PSDA = 1, PIN_EKIN = 3, PIN_VHXC = 4, PIN_FACS = 16, PIN_SIZE = 4096 };
 
-// Device memory for the length of one call that ends with a stream synchronisation: up to 256
-// MiB of the context's own, kept until it is destroyed; more is allocated and freed.  With the
-// scalars in the pinned block instead of copied back (MI355X): two SCF cycles of 108 Al atoms
-// 24.9 -> 23.7 ms, ETRS steps of 64 Si atoms 9.1 -> 8.6 ms, one Hψ of them 305 -> 298 us.
+// Device memory for the length of one call on the context's stream, beside the transform
+// workspace: up to kept_cap() from a block of the context's own, kept until it is destroyed;
+// more is allocated and, once the stream has drained, freed.  p is null where there is no memory.
+// slot: &Ctx::inner inside a call that holds one of &Ctx::call.  With the scalars in the pinned
+// block instead of copied back (MI355X): two SCF cycles of 108 Al atoms 24.9 -> 23.7 ms, ETRS
+// steps of 64 Si atoms 9.1 -> 8.6 ms, one Hψ of them 305 -> 298 us.
 struct CallBuffer {
   void* p = nullptr;
-  CallBuffer(Ctx* c, size_t bytes);
+  CallBuffer(Ctx* c, size_t bytes, Ctx::Kept Ctx::*slot = &Ctx::call);
   ~CallBuffer();
   CallBuffer(const CallBuffer&) = delete;
   CallBuffer& operator=(const CallBuffer&) = delete;
 
  private:
-  bool own = false;
+  Ctx* own = nullptr;  // set if p is to be freed
 };
+// largest block a CallBuffer keeps: 256 MiB or the workspace cap
+size_t kept_cap(const Ctx* c);
 
 // Records the named kernel's launch window when timing is enabled.
 struct TimedLaunch {
@@ -154,9 +157,6 @@ struct TimedLaunch {
 };
 
 void* ws_get(Ctx* ctx, size_t bytes);
-// the context's second workspace, grown on demand like the transform workspace; null if it
-// cannot be allocated.  One call's use of it ends with the call.
-void* aux_get(Ctx* ctx, size_t bytes);
 
 // Set (per host thread) while the multi-cell Hψ graph is being captured: every workspace,
 // table and handle must then already exist, so the growth paths (ws_get, grow), the

@@ -410,7 +410,8 @@ extern "C" int qbh_kinetic_energy(qbh_basis basis, const double* psi_dev, long l
   Ctx* c = ctx_of_basis(basis);
   Basis* b = basis_of(basis);
   hipSetDevice(c->device);
-  double* d = static_cast<double*>(aux_get(c, (nst + kPart + 1) * sizeof(double)));
+  CallBuffer buf(c, (nst + kPart + 1) * sizeof(double));
+  double* d = static_cast<double*>(buf.p);
   if (!d) return sfail(c, QBH_ERR_ALLOC, "kinetic energy scratch");
   hipMemcpyAsync(d, occ, nst * sizeof(double), hipMemcpyHostToDevice, c->stream);
   const dim3 grid = band_grid(b->g.ngw, nst);
