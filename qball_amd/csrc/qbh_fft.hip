@@ -322,8 +322,15 @@ int pipeline_cross(Ctx* ctx, Basis* b, const double* a, long lda, const double* 
   const size_t t1 = c * g.ncol * g.np2, t2 = c * g.np2 * g.nlx * g.np1;
   const size_t per = t1 + (nb + 1) * t2;
   const long N = (long)g.np0 * g.np1 * g.np2;
-  const int S = (int)std::min<size_t>({std::max<size_t>(1, ctx->ws_cap / per), (size_t)nbands, 65535});
+  // slots in flight: up to 2 GiB of T1 and T2, in chunks of about equal size (the current of 128
+  // bands at 72^3 in one, its gradient's 512 columns in two; with 1 GiB in unequal chunks both
+  // calls took 1 % longer), and half as many as long as there is no memory for them
+  const size_t room = std::min<size_t>(ctx->ws_cap, size_t(2) << 30);
+  int S = (int)std::min<size_t>({std::max<size_t>(1, room / per), (size_t)nbands, 65535});
+  const int chunks = (nbands + S - 1) / S;
+  S = (nbands + chunks - 1) / chunks;
   char* ws = static_cast<char*>(ws_get(ctx, S * per));
+  while (!ws && S > 1) ws = static_cast<char*>(ws_get(ctx, (S /= 2) * per));
   // partial grids per slot range: one range at least, more as for the density
   int parts = density_parts(b, S, PREC_FP64, kept_cap(ctx) / nb);
   std::optional<CallBuffer> buf;

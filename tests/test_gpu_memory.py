@@ -60,3 +60,18 @@ def test_small_cap_bounds_what_is_kept(gpu_ctx, cell, what):
     # four fields of one band at a time at most: T1 and T2 of each on this grid
     slot = 16 * (int(np.prod(cell.np[1:])) + N)
     assert kept(cell, call, cap) <= 2 * cap + max(cap, 4 * slot) + SLACK
+
+
+def test_current_of_many_bands_keeps_a_bounded_workspace(gpu_ctx, cell):
+    """Four transforms per band, but at most 2 GiB of them at a time, whatever the cap allows."""
+    import torch
+    nst, g = 700, torch.Generator(device="cuda")
+    g.manual_seed(53)
+    psi = torch.randn(2 * cell.ngw * nst, dtype=torch.float64, device="cuda", generator=g)
+    out = torch.zeros(3 * int(np.prod(cell.np)), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+
+    def call(basis):
+        basis.current(psi.data_ptr(), basis.ngw, nst, np.full(nst, 2.0), 1.0, cell.omega,
+                      j_ptr=out.data_ptr())
+    assert kept(cell, call, 64 << 30) <= (2 << 30) + 2 * 256 * MIB + SLACK
