@@ -357,10 +357,15 @@ static int gram_real(Ctx* c, int n, long K, double* psi, long ld, int* hinfo) {
   // partials, S, W, T and the pivot flag
   CallBuffer buf(c, sizeof(double) * ((slices + 3) * nn + 2));
   double* P = static_cast<double*>(buf.p);
-  // rotated bands, whole or a range of coefficients at a time within the workspace cap
+  // rotated bands, whole or a range of coefficients at a time within the workspace cap (and what
+  // memory there is)
   const size_t room = std::max<size_t>(c->ws_cap / (8 * (size_t)n), 128);
-  const long w = (size_t)K <= room ? K : (long)(room / 128 * 128);
+  long w = (size_t)K <= room ? K : (long)(room / 128 * 128);
   double* out = static_cast<double*>(ws_get(c, sizeof(double) * w * n));
+  while (!out && w > 128) {
+    w = std::max(w / 256 * 128, 128L);
+    out = static_cast<double*>(ws_get(c, sizeof(double) * w * n));
+  }
   if (!P || !out) return dfail(c, QBH_ERR_ALLOC, "gram scratch allocation failed");
   double* S = P + slices * nn;
   double* W = S + nn;
