@@ -105,7 +105,7 @@ extern "C" int qbh_ctx_create(int device, void* stream, qbh_ctx* out) {
     }
     h->c.own_stream = true;
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&h->c.pin), PIN_SIZE * sizeof(double)) != hipSuccess) {
+  if (!ctx_acquire(&h->c)) {
     if (h->c.own_stream) hipStreamDestroy(h->c.stream);
     delete h;
     return QBH_ERR_ALLOC;
@@ -117,27 +117,34 @@ extern "C" int qbh_ctx_create(int device, void* stream, qbh_ctx* out) {
 
 namespace qbh {
 void blas_destroy(Ctx* c);
+
+bool ctx_acquire(Ctx* c) {
+  return hipHostMalloc(reinterpret_cast<void**>(&c->pin), PIN_SIZE * sizeof(double)) == hipSuccess;
 }
+
+void ctx_release(Ctx* c) {
+  for (auto& r : c->timer.pending) {
+    hipEventDestroy(r.a);
+    hipEventDestroy(r.b);
+  }
+  blas_destroy(c);  // rocBLAS handle and hipBLASLt state
+  if (c->side) {
+    hipStreamSynchronize(c->side);
+    hipStreamDestroy(c->side);
+  }
+  if (c->ev_fork) hipEventDestroy(c->ev_fork);
+  if (c->ev_join) hipEventDestroy(c->ev_join);
+  for (void* p : {c->ws, c->call.p, c->inner.p})
+    if (p) hipFree(p);
+  if (c->pin) hipHostFree(c->pin);
+}
+}  // namespace qbh
 
 extern "C" int qbh_ctx_destroy(qbh_ctx ctx) {
   if (!ctx) return QBH_ERR_ARG;
   hipSetDevice(ctx->c.device);
   hipStreamSynchronize(ctx->c.stream);
-  for (auto& r : ctx->c.timer.pending) {
-    hipEventDestroy(r.a);
-    hipEventDestroy(r.b);
-  }
-  qbh::blas_destroy(&ctx->c);
-  if (ctx->c.side) {
-    hipStreamSynchronize(ctx->c.side);
-    hipStreamDestroy(ctx->c.side);
-  }
-  if (ctx->c.ev_fork) hipEventDestroy(ctx->c.ev_fork);
-  if (ctx->c.ev_join) hipEventDestroy(ctx->c.ev_join);
-  if (ctx->c.ws) hipFree(ctx->c.ws);
-  for (const qbh::Ctx::Kept* k : {&ctx->c.call, &ctx->c.inner})
-    if (k->p) hipFree(k->p);
-  if (ctx->c.pin) hipHostFree(ctx->c.pin);
+  ctx_release(&ctx->c);
   if (ctx->c.own_stream) hipStreamDestroy(ctx->c.stream);
   delete ctx;
   return QBH_OK;

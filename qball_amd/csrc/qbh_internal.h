@@ -122,6 +122,12 @@ struct Ctx {
   std::string scratch_err;
 };
 
+// What every context needs besides its stream, the caller's or a branch's (device current):
+// ctx_acquire allocates the pinned block (false: no memory), ctx_release frees everything but
+// the stream, which has drained.
+bool ctx_acquire(Ctx* c);
+void ctx_release(Ctx* c);
+
 // Looks up (once per device, with `device` current) the device address of the
 // allocation-free scratch array and stores it in c->scratch (qbh_api.hip).
 void noalloc_scratch_setup(Ctx* c);

@@ -263,11 +263,7 @@ struct qbh_batch_s {
 };
 
 static void destroy_branch(Ctx* b) {
-  blas_destroy(b);  // rocBLAS handle and hipBLASLt state
-  if (b->ws) hipFree(b->ws);
-  if (b->side) hipStreamDestroy(b->side);
-  if (b->ev_fork) hipEventDestroy(b->ev_fork);
-  if (b->ev_join) hipEventDestroy(b->ev_join);
+  ctx_release(b);
   if (b->stream) hipStreamDestroy(b->stream);
   delete b;
 }
@@ -353,6 +349,10 @@ extern "C" int qbh_batch_create(qbh_ctx ctx, int ncells, const qbh_ham* hams,
       return ufail(uc, QBH_ERR_DEVICE, "branch stream creation failed");
     }
     c->own_stream = true;
+    if (!ctx_acquire(c)) {
+      qbh_batch_destroy(bt);
+      return ufail(uc, QBH_ERR_ALLOC, "branch context allocation failed");
+    }
   }
   // eager pass: allocates every workspace, table and scratch buffer the graph will use
   int r = QBH_OK;
