@@ -182,6 +182,11 @@ static const PlaneOps* plane_ops(const Basis* b, int prec) {
   return r && r->plane.fits && r->plane.fits(g) ? &r->plane : nullptr;
 }
 
+// row transforms of a plane (n rows of nlx lines) per wavefront
+static long plane_work(const GridDev& g, const PlaneOps* p) {
+  return (long)g.np0 * g.nlx * p->wgs / 8;
+}
+
 // slots per plane workgroup: as many as leave 2048 workgroups (72^3, 128 complex bands: 1, 2,
 // 4, 8 slots 360, 330, 320, 346 us; 64^3, 128 real bands 108, 100, 98, 97)
 static int plane_spw(const Basis* b, int nslots) {
@@ -248,8 +253,13 @@ int pipeline_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, in
 
 // Slot ranges of the density x pass for chunks of nslots slots: each workgroup sums all slots
 // of its rows, so the rows alone give np2 * np1 / rows-per-workgroup workgroups (216 at 72^3,
-// 1260 at 140^3: 2.5 rounds of two per CU).  Ranges for about 4096 workgroups, at least 4
-// slots each, with at most cap_bytes of partial grids.
+// 1260 at 140^3: 2.5 rounds of two per CU).  Ranges for about 4096 workgroups, with at most
+// cap_bytes of partial grids; a range costs a partial grid written and read, so it takes at
+// least 4 slots, and 16 where the rows alone fill the chip and it only evens out the last
+// round.  One range against n, density with its z and y passes (MI355X, FP64 unless noted):
+// 36 x 42 x 36, 32 slots 87 -> 52 us (8); 72 x 84 x 72, 128 slots 471 -> 345 (14); 108^3, 128
+// slots 996 -> 930 (7); 140^3, 400 slots 6.45 -> 6.27 ms (4), 32 slots 561 -> 553 us (2; FP32 339
+// -> 330), with 4 561 (339); 8 slots 167 us (FP32 112), with 2 181 (121).
 static int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
   const GridDev& g = b->g;
   const EdgeOps* r = b->tune.x_reg ? register_ops(g.np0, prec) : nullptr;
@@ -257,21 +267,28 @@ static int density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes)
   const long rows = (long)g.np2 * ((g.np1 + yb - 1) / yb);
   const long N = (long)g.np0 * g.np1 * g.np2;
   long p = std::min<long>((4096 + rows - 1) / rows, 16);
-  p = std::min<long>({p, nslots / 4, (long)(cap_bytes / (8 * (size_t)N))});
+  p = std::min<long>({p, nslots / (rows < 512 ? 4 : 16), (long)(cap_bytes / (8 * (size_t)N))});
   return (int)std::max<long>(p, 1);
 }
 
 // The same for the plane form, whose workgroups are few and long: of up to 16 ranges the number
-// with the fewest slots times rounds of resident workgroups, the smaller one if equal.  Density
-// without z passes, passes -> plane: 24^3, 16 real bands 23 -> 15 us; 64^3, 128 real bands 98 ->
-// 66; 72^3, 64 complex bands 136 -> 122; 88^3, 100 real bands 231 -> 196.
+// with the least time for its rounds of resident workgroups and its partial grids, the smaller
+// one if equal.  A slot of a plane takes about 1.5 us and 14 ns per n * nlx / wavefronts (36^3
+// 4 us, 72^3 10.5, 90^3 8, 100^3 10), a range 16 bytes a point at 4.5 TB/s, and the sum of the
+// partial grids one more and a launch (4 us).  Density without z passes, passes -> plane: 24^3,
+// 16 real bands 23 -> 15 us; 64^3, 128 real bands 98 -> 66; 72^3, 64 complex bands 136 -> 122;
+// 88^3, 100 real bands 231 -> 196.  Against the fewest rounds alone, whole density: 100^3, 16
+// slots 172 -> 133 us (2 ranges, not 16); 90^3, 8 slots 88 -> 82 (2, not 8).
 static int plane_parts(const Basis* b, const PlaneOps* p, int nslots, size_t cap_bytes) {
   const GridDev& g = b->g;
   const size_t grid = 8 * (size_t)g.np0 * g.np1 * g.np2;
   const long most = std::min<long>({16, nslots, (long)(cap_bytes / grid)});
-  long best = 1, cost = 0;
+  const double slot = 1.5 + 0.014 * plane_work(g, p);
+  long best = 1;
+  double cost = 0.0;
   for (long k = 1; k <= most; ++k) {
-    const long c = (g.np2 * k + 256L * p->wgs - 1) / (256L * p->wgs) * ((nslots + k - 1) / k);
+    const double c = (g.np2 * k + 256L * p->wgs - 1) / (256L * p->wgs) * ((nslots + k - 1) / k) * slot +
+                     (k > 1 ? 4.0 + (k + 1) * 2.0 * grid / 4.5e6 : 0.0);
     if (k == 1 || c < cost) {
       best = k;
       cost = c;
