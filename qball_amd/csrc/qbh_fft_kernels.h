@@ -586,10 +586,16 @@ k_xpass(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   }
   if (OP == X_DENSITY) {
     double* o = out + blockIdx.y * N + grow0;
+    const bool one = gridDim.y == 1;  // one slot range: accumulate
 #pragma unroll
     for (int k = 0; k < EPL; ++k) {
       const int e = lane + k * 64;
-      if (e < nel) o[e] = gridDim.y > 1 ? acc[k] : o[e] + acc[k];
+      if (one && e < nel) acc[k] += o[e];
+    }
+#pragma unroll
+    for (int k = 0; k < EPL; ++k) {
+      const int e = lane + k * 64;
+      if (e < nel) o[e] = acc[k];
     }
   }
 }
@@ -941,16 +947,19 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   }
   if (OP == X_DENSITY) {
     double* o = out + (long)blockIdx.y * n * np1 * np2 + grow0;
+    const bool one = gridDim.y == 1;  // one slot range: accumulate
 #pragma unroll
     for (int ib = 0; ib < IB; ++ib) {
       const int t = lane + 64 * ib;
       const int r = t / N1, k1 = t % N1;
       if (t < TB && r < nyl) {
+        double* e = o + r * n + k1;
+        if (one) {  // (a lane's loads in flight together)
 #pragma unroll
-        for (int k2 = 0; k2 < N2; ++k2) {
-          double* e = o + r * n + k1 + N1 * k2;
-          *e = gridDim.y > 1 ? acc[ib][k2] : *e + acc[ib][k2];
+          for (int k2 = 0; k2 < N2; ++k2) acc[ib][k2] += e[N1 * k2];
         }
+#pragma unroll
+        for (int k2 = 0; k2 < N2; ++k2) e[N1 * k2] = acc[ib][k2];
       }
     }
   }
