@@ -173,18 +173,36 @@ static int xpass_t(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* in, 
   return check_launch(ctx, name);
 }
 
-// plane forms for this basis and precision, or null.  FP32 keeps the passes: the plane's
-// forward y transform has another radix order, which rounds differently.
-static const PlaneOps* plane_ops(const Basis* b, int prec) {
-  const GridDev& g = b->g;
-  if (prec != PREC_FP64 || g.np0 != g.np1 || !b->tune.zy_reg || !b->tune.x_reg) return nullptr;
-  const EdgeOps* r = register_ops(g.np0, prec);
-  return r && r->plane.fits && r->plane.fits(g) ? &r->plane : nullptr;
-}
-
 // row transforms of a plane (n rows of nlx lines) per wavefront
 static long plane_work(const GridDev& g, const PlaneOps* p) {
   return (long)g.np0 * g.nlx * p->wgs / 8;
+}
+
+// plane forms of the call `use` for nslots slots of this basis and precision, or null.  FP32 keeps
+// the passes: the plane's forward y transform has another radix order, which rounds differently.
+//
+// A plane is one chain of dependent stages in one workgroup; the passes take three launches instead
+// and spread the same work over more workgroups.  So the plane pays where its chain is short
+// (transforms and density: four rounds, or 1300 row elements per SIMD; Hψ, which saves one more
+// launch: 2100, or 2600 in spheres up to half the edge), or where there are enough planes for
+// their work.
+// Passes against plane, one slot, cubes (MI355X): Hψ 64^3 nlx 31 30 -> 25 us, 48^3 nlx 37 29 -> 29,
+// 60^3 nlx 45 33 -> 38, 60^3 nlx 57 36 -> 46; backward 64^3 nlx 31 (4 rounds) 17 -> 14, 60^3 nlx 29
+// (6) 15 -> 17, 48^3 nlx 45 (6) 16 -> 20; forward 54^3 nlx 27 (4) 19 -> 16, 60^3 nlx 45 (7) 20 -> 24;
+// density 64^3 nlx 31 37 -> 34, 72^3 nlx 35 (7) 38 -> 40; with four slots Hψ of 60^3 nlx 45 51 -> 46.
+// Stores of fat spheres on the longest edges pay at no count (60^3 nlx 57, 64 slots 232 -> 261).
+enum PlaneUse { PLANE_VMUL, PLANE_STORE, PLANE_LOAD, PLANE_DENSITY };
+static const PlaneOps* plane_ops(const Basis* b, int prec, int nslots, PlaneUse use) {
+  const GridDev& g = b->g;
+  if (prec != PREC_FP64 || g.np0 != g.np1 || !b->tune.zy_reg || !b->tune.x_reg) return nullptr;
+  const EdgeOps* r = register_ops(g.np0, prec);
+  if (!r || !r->plane.fits || !r->plane.fits(g)) return nullptr;
+  const long work = 4 * plane_work(g, &r->plane);
+  const bool alone = use == PLANE_VMUL ? work <= (g.nlx <= g.np0 / 2 + 1 ? 2600 : 2100)
+                                       : work <= 1300 || r->plane.rounds(g) <= 4;
+  if (!alone && work > 21L * g.np2 * nslots) return nullptr;
+  if (use == PLANE_STORE && work > 2700 && 8 * g.nlx > 5 * g.np0) return nullptr;
+  return &r->plane;
 }
 
 // slots per plane workgroup: as many as leave 2048 workgroups (72^3, 128 complex bands: 1, 2,
@@ -208,7 +226,7 @@ static int plane_pass(Ctx* ctx, Basis* b, const PipelineArgs& a, PlaneOps::Launc
 
 int pipeline_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v, double* out,
                   long ldo, const double* kin, int store) {
-  if (const PlaneOps* p = plane_ops(b, a.prec)) {
+  if (const PlaneOps* p = plane_ops(b, a.prec, a.nslots, PLANE_VMUL)) {
     if (int e = bwd_z(ctx, b, a)) return e;
     if (int e = plane_pass(ctx, b, a, p->vmul, plane_spw(b, a.nslots), v, nullptr, nullptr, 0, 1.0,
                            "plane_vmul"))
@@ -223,7 +241,7 @@ int pipeline_vmul(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* v, do
 }
 
 int pipeline_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f) {
-  if (const PlaneOps* p = plane_ops(b, a.prec); p && p->store) {
+  if (const PlaneOps* p = plane_ops(b, a.prec, a.nslots, PLANE_STORE); p && p->store) {
     if (int e = bwd_z(ctx, b, a)) return e;
     return plane_pass(ctx, b, a, p->store, plane_spw(b, a.nslots), nullptr, f, nullptr, 0, 1.0,
                       "plane_store");
@@ -237,7 +255,7 @@ int pipeline_store(Ctx* ctx, Basis* b, const PipelineArgs& a, double* f) {
 int pipeline_load(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* f, int real_input,
                   double scale, double* out, long ldo) {
   int e;
-  if (const PlaneOps* p = plane_ops(b, a.prec); p && p->load) {
+  if (const PlaneOps* p = plane_ops(b, a.prec, a.nslots, PLANE_LOAD); p && p->load) {
     e = plane_pass(ctx, b, a, real_input ? p->load_real : p->load, plane_spw(b, a.nslots), f,
                    nullptr, nullptr, 0, scale, "plane_load");
     return e ? e : fwd_z(ctx, b, a, out, ldo, nullptr, 1);
@@ -298,7 +316,7 @@ static int plane_parts(const Basis* b, const PlaneOps* p, int nslots, size_t cap
 }
 
 int pipeline_density_parts(const Basis* b, int nslots, int prec, size_t cap_bytes) {
-  const PlaneOps* p = plane_ops(b, prec);
+  const PlaneOps* p = plane_ops(b, prec, nslots, PLANE_DENSITY);
   return p ? plane_parts(b, p, nslots, cap_bytes) : density_parts(b, nslots, prec, cap_bytes);
 }
 
@@ -309,7 +327,7 @@ int pipeline_density(Ctx* ctx, Basis* b, const PipelineArgs& a, const double* de
   const int parts = (a.nslots + spw - 1) / spw;
   double* out = parts > 1 ? a.dens_part : rho;
   int r;
-  if (const PlaneOps* p = plane_ops(b, a.prec)) {
+  if (const PlaneOps* p = plane_ops(b, a.prec, a.nslots, PLANE_DENSITY)) {
     if (int e = bwd_z(ctx, b, a)) return e;
     r = plane_pass(ctx, b, a, p->density, spw, nullptr, out, dens, cd, 1.0, "plane_density");
   } else {

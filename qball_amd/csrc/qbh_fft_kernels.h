@@ -1383,6 +1383,7 @@ struct PlaneOps {
                           const double* in, double* out, const double* dens, int cplx_density,
                           double scale);
   bool (*fits)(const GridDev& g) = nullptr;
+  int (*rounds)(const GridDev& g) = nullptr;  // dependent rounds of one direction (plane_rounds)
   int wgs = 0;  // workgroups per compute unit
   Launch vmul = nullptr, density = nullptr;
   Launch store = nullptr, load = nullptr, load_real = nullptr;  // null: separate passes

@@ -349,6 +349,15 @@ bool plane_fits(const GridDev& g) {
   return Plane<N1, N2>::WGS * Plane<N1, N2>::lds(g.nlx) <= 163840;
 }
 
+// rounds of tasks that follow one another in the workgroup for one direction of a plane: the
+// two stages of the y transforms (nlx lines) and the row groups of the x transforms
+template <int N1, int N2>
+int plane_rounds(const GridDev& g) {
+  using C = Plane<N1, N2>;
+  constexpr int NT = C::NW * 64, R = C::NW * C::LPW;
+  return (g.nlx * N1 + NT - 1) / NT + (g.nlx * N2 + NT - 1) / NT + (C::n + R - 1) / R;
+}
+
 template <int OP, int N1, int N2>
 void launch_plane(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
                   const double* in, double* out, const double* dens, int cplx_density,
@@ -370,6 +379,7 @@ constexpr PlaneOps plane_edge() {
   PlaneOps p;
   if constexpr (sizeof(T) == 8 && N1 * N2 <= 108) {
     p.fits = plane_fits<N1, N2>;
+    p.rounds = plane_rounds<N1, N2>;
     p.wgs = Plane<N1, N2>::WGS;
     p.vmul = launch_plane<X_VMUL, N1, N2>;
     p.density = launch_plane<X_DENSITY, N1, N2>;

@@ -397,3 +397,54 @@ def test_fp32_forward_error(gpu_ctx, n):
         assert err[1][k] <= 1.02 * err[0][k], err
     ham.close()
     basis.close()
+
+
+@pytest.mark.parametrize("nb,vmul,store,load,density", [
+    (1, False, False, False, False), (3, False, False, False, False), (8, True, True, True, True)])
+@pytest.mark.parametrize("n", (54, 56))
+def test_plane_needs_enough_planes(gpu_ctx, n, nb, vmul, store, load, density):
+    """A sphere that fills most of the plane (nlx = 43): few slots take the passes, which spread
+    one slot over the chip, more take the plane kernel; the oracle's results either way."""
+    import torch
+    from oracle import fft as offt
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=170.0, nbands=nb, seed=47)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut), n, n, 50)
+    r, c = sysm.rods, sysm.psi
+    basis = Basis(gpu_ctx, True, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], (n, n, 50),
+                  sysm.b)
+    N, cd, nslots = basis.N, to_dev(c), (nb + 1) // 2
+    rng = np.random.default_rng(n)
+    v = rng.standard_normal(N)
+    vd, hd, back = real_to_dev(v), torch.zeros_like(cd), torch.zeros_like(cd)
+    f = torch.zeros(2 * nslots * N, dtype=torch.float64, device="cuda")
+    rho = torch.zeros(N, dtype=torch.float64, device="cuda")
+    ham = Hamiltonian(gpu_ctx, basis)
+    ham.set_vloc(vd.data_ptr())
+    torch.cuda.synchronize()
+    gpu_ctx.timing_report()
+    gpu_ctx.set_timing(True)
+    ham.hpsi(cd.data_ptr(), basis.ngw, nb, sysm.occ, hd.data_ptr(), basis.ngw, flags=0x4)
+    basis.backward(cd.data_ptr(), basis.ngw, nb, True, f.data_ptr())
+    basis.forward(f.data_ptr(), nb, True, back.data_ptr(), basis.ngw)
+    basis.density(cd.data_ptr(), basis.ngw, nb, sysm.occ, 1.0, sysm.omega, rho.data_ptr())
+    gpu_ctx.sync()
+    ran = gpu_ctx.timing_report()
+    gpu_ctx.set_timing(False)
+    assert ["plane_" + k in ran for k in ("vmul", "store", "load", "density")] == \
+        [vmul, store, load, density]
+    ref = oh.rs_mul_add(maps, c, v, np.zeros_like(c))
+    assert rel_err(from_dev(hd, basis.ngw, nb), ref) <= 1e-12
+    fg = f.cpu().numpy().view(np.complex128).reshape(nslots, N)
+    for s in range(nslots):
+        two = 2 * s + 1 < nb
+        ref = offt.backward(maps, c[:, 2 * s], c[:, 2 * s + 1] if two else None)
+        assert rel_err(fg[s], ref.ravel()) <= 1e-12
+    assert rel_err(from_dev(back, basis.ngw, nb), c) <= 1e-12
+    assert rel_err(rho.cpu().numpy(),
+                   oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)) <= 1e-12
+    ham.close()
+    basis.close()
