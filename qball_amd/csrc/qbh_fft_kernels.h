@@ -126,8 +126,13 @@ template <typename T, int N1, int N2> struct YCfg {
   static constexpr int ZB = NWAVE * LPW / LB;
 };
 
-// x pass: line elements per thread of the short variant, for spheres up to half the edge
+// x pass: line elements per thread of the short variant, for spheres up to half the edge, and of
+// the middle one, for up to eight lines more, of the potential multiply and the density
+// (registers per element; with the full count, which the middle one avoids, 180^3 with 97 lines,
+// 64 bands: Hψ 2.80 ms against 2.55; with the middle count in place of the short one 160^3, 79
+// lines: density 0.94 against 0.88 ms)
 constexpr int x_short(int n, int yb) { return (yb * (n / 2) + NTHR - 1) / NTHR; }
+constexpr int x_middle(int n, int yb) { return (yb * (n / 2 + 8) + NTHR - 1) / NTHR; }
 
 template <typename T>
 __device__ __forceinline__ const cplx<T>* twtab(const GridDev& g, int axis);
@@ -650,8 +655,8 @@ k_xpass2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
   // factors twiddle_row forms, computed once instead of per slot (measured at
   // 140 = 14*10: x pass 6.24 -> 6.01 ms per FP64 Hψ).  Not for the FP64 kernels with the
   // full line-element count, which have no registers to spare.
-  constexpr int GS = x_short(n, YB);
-  constexpr bool TWB = QBH_XTWB && (sizeof(T) == 4 || GPW <= GS) && !stockham_order<T, N1, N2>();
+  constexpr int GT = LPW == 4 ? x_middle(n, YB) : x_short(n, YB);
+  constexpr bool TWB = QBH_XTWB && (sizeof(T) == 4 || GPW <= GT) && !stockham_order<T, N1, N2>();
   cplx<T> twb[IB][TWB ? N2 - 1 : 1];
   if constexpr (TWB && OP == X_VMUL) {
 #pragma unroll
@@ -1480,8 +1485,8 @@ void launch_yfwd(hipStream_t st, const GridDev& g, const PipelineArgs& a) {
       g, static_cast<const cplx<T>*>(a.t2), static_cast<cplx<T>*>(a.t1));
 }
 
-// register x pass; line elements per thread: a short count for spheres up to about half the
-// edge (the usual Hψ grid), the full edge otherwise
+// register x pass; line elements per thread: a short count for spheres up to half the edge (the
+// usual Hψ grid), a middle one for a few lines more, the full edge otherwise
 template <typename T, int OP, int N1, int N2>
 void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw, const double* in,
                double* out, const double* dens, int cplx_density) {
@@ -1492,8 +1497,13 @@ void launch_x2(hipStream_t st, const GridDev& g, const PipelineArgs& a, int spw,
   const size_t lds =
       sizeof(cplx<T>) * ((size_t)n + (size_t)YB * Pad<N1, N2, QBH_XLDS_PAD>::row(n) + NTHR);
   auto* t2 = static_cast<cplx<T>*>(a.t2);
-  if ((g.nlx * YB + NTHR - 1) / NTHR <= GS)
+  constexpr int GM = OP == X_VMUL || OP == X_DENSITY ? x_middle(n, YB) : GS;
+  const int need = (g.nlx * YB + NTHR - 1) / NTHR;
+  if (need <= GS)
     k_xpass2<T, OP, N1, N2, GS><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, in, out, dens,
+                                                         cplx_density);
+  else if (GM < GF && need <= GM)
+    k_xpass2<T, OP, N1, N2, GM><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, in, out, dens,
                                                          cplx_density);
   else
     k_xpass2<T, OP, N1, N2, GF><<<grid, NTHR, lds, st>>>(g, t2, a.nslots, spw, in, out, dens,

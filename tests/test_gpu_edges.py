@@ -448,3 +448,40 @@ def test_plane_needs_enough_planes(gpu_ctx, n, nb, vmul, store, load, density):
                    oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)) <= 1e-12
     ham.close()
     basis.close()
+
+
+@pytest.mark.parametrize("grid,ecut,nlx,real,nb", [
+    ((32, 18, 24), 25.0, 17, True, 3), ((36, 30, 28), 60.0, 25, False, 2),
+    ((72, 50, 44), 170.0, 43, True, 2), ((128, 66, 70), 395.0, 65, True, 3)])
+def test_spheres_just_past_half_the_edge(gpu_ctx, grid, ecut, nlx, real, nb):
+    """Local Hψ and density of spheres of a few lines more than half the edge (the x pass'
+    middle count of line elements), long and short edges."""
+    import torch
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=ecut, nbands=nb, seed=48, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), *grid)
+    assert 2 * int(np.abs(sysm.idx[:, 0]).max()) + 1 == nlx and grid[0] < 2 * nlx < grid[0] + 18
+    r, c = sysm.rods, sysm.psi
+    basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"], grid, sysm.b)
+    v = np.random.default_rng(nlx).standard_normal(basis.N)
+    vd, cd = real_to_dev(v), to_dev(c)
+    hd = torch.zeros_like(cd)
+    ham = Hamiltonian(gpu_ctx, basis)
+    ham.set_vloc(vd.data_ptr())
+    ref = oh.rs_mul_add(maps, c, v, np.zeros_like(c))
+    rho_ref = oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)
+    for flags, tol in ((0, 1e-12), (0x10, 2e-6)):
+        rho = torch.zeros(basis.N, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        ham.hpsi(cd.data_ptr(), basis.ngw, nb, sysm.occ, hd.data_ptr(), basis.ngw,
+                 flags=0x4 | flags)
+        basis.density(cd.data_ptr(), basis.ngw, nb, sysm.occ, 1.0, sysm.omega, rho.data_ptr(),
+                      flags)
+        gpu_ctx.sync()
+        assert rel_err(from_dev(hd, basis.ngw, nb), ref) <= tol
+        assert rel_err(rho.cpu().numpy(), rho_ref) <= tol
+    ham.close()
+    basis.close()
