@@ -4,9 +4,11 @@
 
 namespace qbh {
 
-// Slices the reduction of an R x C output with reduction length Q is cut into (want > 0:
-// that many, else enough for ~2048 workgroups, each slice at least 512 long); the count
-// actually used (every slice non-empty).
+// Slices the reduction of an R x C output with reduction length Q is cut into, at most 64; the
+// count actually used (every slice non-empty).  want > 0: that many, each slice at least 512
+// long.  Else FP32: enough for about 2048 workgroups of the 128 x 128 tile, each slice at least
+// 512 long, whatever the tile; FP64: the same with that tile, and the cheapest count with a
+// smaller one, slices down to 64 long (tile_cost).
 int mfma_slices(bool fp32, int R, int C, long Q, int want);
 // Length of each slice for `slices` slices (a multiple of the 16-element stage).
 long mfma_slice_len(long Q, int slices);
@@ -33,5 +35,10 @@ int mfma_gemm_sym(hipStream_t st, int R, long Q, const double* X, long ldx, doub
 // Y[c + q ldy], q < R (as mfma_gemm_qc without the zero half of the reduction; O apart from Y).
 int mfma_gemm_tri(hipStream_t st, int R, int C, const double* X, long ldx, const double* Y,
                   long ldy, double* O, long ldo);
+
+// Width of the tiles (32, 64, 128), and the slices, of a product of these sizes under the
+// built-in rule, for the tests: which 0, 1: F in FP64, FP32 (mfma_gemm_qq); 2, 3: βF
+// (mfma_gemm_qc; mfma_gemm_tri is as 2); 4: the symmetric product (C = R).
+extern "C" int qbh_product_tile(int which, int R, int C, long Q, int* slices);
 
 }  // namespace qbh

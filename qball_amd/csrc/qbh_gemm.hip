@@ -566,7 +566,13 @@ __global__ void __launch_bounds__(kThreads, TB == 4 ? 2 : 4) k_gemm_direct(Args 
 // has the most MFMAs per loaded element, the smaller ones waste less on edges and make enough
 // workgroups for small outputs), some 80 elements more for its start and end, and a fifth more
 // when it is alone on its CU.  The 256 CUs share the workgroups, and each slice's partial
-// output is written and read once.
+// output is written and read once.  Four 64 x 64 tiles share a CU, so in FP64 F the uneven end
+// costs them a workgroup more where few long slices fall to a CU (1320 projectors, 900 bands, 57052
+// reals: 4, 8, 16, 24 slices 3.13, 2.64, 2.57, 2.51 ms, large tile with 24 2.86).  FP32 slices over
+// 5000 long let the workgroups that share operands drift apart in cache, which costs the small
+// tiles a third (1600 rows, 390 bands, 40 slices of 7270: 4.73 ms against 4.33 on the large one,
+// and βF right after it 3.7 against 3.3).  Over 336 measured shapes F is nowhere more than 3 %
+// slower than with the large tile, βF never.
 //   form                          us(4)   us(2)   us(1)
 //   FP64 F, through LDS           0.140   0.038   0.0115
 //   FP64 Hψ += βF, direct         0.122   0.045   0.022
@@ -590,10 +596,14 @@ inline long tiles_of(int R, int C, int tb) {
 double tile_cost(Form f, int R, int C, long Q, int tb, long slices) {
   static const double us[3][3] = {{0.140, 0.038, 0.0115}, {0.122, 0.045, 0.022},
                                   {0.070, 0.0187, 0.0056}};
-  const long per_cu = (tiles_of(R, C, tb) * slices + 255) / 256;
-  const double u = us[f][tb == 4 ? 0 : tb == 2 ? 1 : 2] * (per_cu == 1 ? 1.2 : 1.0);
+  const double len = (double)Q / slices;
+  const long wgs = tiles_of(R, C, tb) * slices, per_cu = (wgs + 255) / 256;
+  double rounds = per_cu == 1 ? 1.2 : per_cu;
+  if (tb == 2 && f == FORM_LDS64 && wgs > 1024 && len > 3000)
+    rounds = std::max(rounds, 0.9 * wgs / 256 + 1.2);
+  if (tb < 4 && f == FORM_LDS32 && slices > 1 && len > 5000) rounds *= 1.35;
   const double bytes = slices > 1 ? 2.0 * slices * R * (double)C * (f == FORM_LDS32 ? 4 : 8) : 0.0;
-  return per_cu * u * ((double)Q / slices + 80) + bytes / 4e6;
+  return rounds * us[f][tb == 4 ? 0 : tb == 2 ? 1 : 2] * (len + 80) + bytes / 4e6;
 }
 
 template <typename T, bool YC, bool OUTC, int TB>
@@ -738,6 +748,20 @@ int mfma_gemm_qc(hipStream_t st, bool fp32, int R, int C, long Q, const void* X,
   a.accumulate = accumulate ? 1 : 0;
   launch<true, true>(a, st, fp32, 1, best_tile(fp32 ? FORM_LDS32 : FORM_DIRECT64, R, C, Q, 1));
   return 0;
+}
+
+extern "C" int qbh_product_tile(int which, int R, int C, long Q, int* slices) {
+  const bool fp32 = which & 1;
+  int s = 1;
+  Form f = fp32 ? FORM_LDS32 : FORM_LDS64;
+  if (which < 2)
+    s = mfma_slices(fp32, R, C, Q, 0);
+  else if (which == 4)
+    s = mfma_sym_slices(R, Q);
+  else if (!fp32)
+    f = FORM_DIRECT64;
+  if (slices) *slices = s;
+  return 32 * best_tile(f, R, C, Q, s);
 }
 
 // slices of the symmetric product: from eight 128 x 128 tiles on, as many as one round of two

@@ -101,3 +101,32 @@ int main() {
     rc, enl, msg = subprocess.run([exe], check=True, capture_output=True,
                                   text=True).stdout.split()
     assert int(rc) != 0 and float(enl) != 42.0 and int(msg) > 0
+
+
+def product_tile(which, R, C, Q):
+    from qball_amd import lib
+    s = ctypes.c_int()
+    f = lib().qbh_product_tile
+    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long,
+                  ctypes.POINTER(ctypes.c_int)]
+    return f(which, R, C, Q, ctypes.byref(s)), s.value
+
+
+@pytest.mark.parametrize("which,R,C,Q,tile,slices", [
+    # measured slower on 64-wide tiles: FP32 slices of 5500 to 9088 (F and the product after it),
+    # FP64 with few workgroups a CU (4 slices 3.13 ms, large tile with 24 2.86)
+    (1, 1600, 300, 290810, 128, 53), (1, 1600, 390, 290810, 128, 40),
+    (1, 1600, 520, 290810, 128, 32), (0, 1320, 900, 57052, None, 8), (0, 2048, 300, 145406, None, 16),
+    # faster on small tiles
+    (0, 32, 16, 2302, 32, 29), (0, 256, 128, 18278, 32, 16), (1, 256, 128, 18278, 32, 35),
+    (1, 1560, 390, 145406, 64, 40), (0, 1320, 200, 57052, 64, 24), (2, 16, 2302, 32, 32, 1),
+    # as fast on the large tile
+    (0, 2048, 1024, 145838, 128, 16), (2, 1024, 145838, 2048, 128, 1), (4, 1024, 1024, 145838, 128, 14)])
+def test_product_tiles(which, R, C, Q, tile, slices):
+    """Tile and slice rule of the matrix-core products at measured shapes (None: either tile,
+    with at least that many slices)."""
+    got = product_tile(which, R, C, Q)
+    if tile is None:
+        assert got[1] >= slices
+    else:
+        assert got == (tile, slices)
