@@ -78,3 +78,14 @@ def synthetic_spdf():
         phi.append((r ** (l + 1)) * np.exp(-0.8 * r * r))
     return {"zval": zv, "lmax": lmax, "llocal": llocal, "deltar": 0.01, "vps": vps,
             "phi": phi, "nquad": 0}
+
+
+def product_tile(which, R, C, Q):
+    """Tile width and slices of a matrix-core product under the built-in rule (qbh_gemm.h)."""
+    import ctypes
+    from qball_amd import lib
+    s = ctypes.c_int()
+    f = lib().qbh_product_tile
+    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long,
+                  ctypes.POINTER(ctypes.c_int)]
+    return f(which, R, C, Q, ctypes.byref(s)), s.value

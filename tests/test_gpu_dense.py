@@ -63,3 +63,42 @@ def test_gram_padding_small_workspace_and_singular(cell):
     assert torch.equal(cd, before)
     basis.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("nst,sym,tri", [(385, 32, 64), (640, 128, 128), (768, 64, 128),
+                                         (900, 128, 128)])
+def test_gram_wide_tiles(gpu_ctx, nst, sym, tri):
+    """The 64 and 128 wide tiles of the symmetric and the triangular product over several tile
+    rows and slices, with the tiles that ran (same bar: 900 bands, condition of L 11)."""
+    from helpers import make_gpu_basis, product_tile
+    from oracle import hpsi as oh
+    from qball_amd.workload import make_system
+    big = make_system(ncell=1, ecut_ry=60.0, nbands=nst, seed=41)
+    K = 2 * big.ngw
+    assert product_tile(4, nst, nst, K)[0] == sym and product_tile(2, nst, K, nst)[0] == tri
+    basis = make_gpu_basis(gpu_ctx, big)
+    cd = to_dev(big.psi)
+    basis.gram(cd.data_ptr(), basis.ngw, nst)
+    gpu_ctx.sync()
+    got = from_dev(cd, basis.ngw, nst)
+    assert rel_err(got, oh.gram(big.psi, True)) <= 1e-11
+    basis.close()
+
+
+@pytest.mark.parametrize("nst", [1, 16, 70, 129])
+def test_gram_of_bands_at_an_odd_double(gpu_ctx, cell, nst):
+    """A psi aligned to 8 bytes only, which the matrix-core products do not read (rocBLAS and
+    rocSOLVER): the same bands."""
+    import torch
+    from helpers import make_gpu_basis
+    from oracle import hpsi as oh
+    c = cell.psi[:, :nst]
+    basis = make_gpu_basis(gpu_ctx, cell)
+    buf = torch.zeros(2 * cell.ngw * nst + 1, dtype=torch.float64, device="cuda")
+    buf[1:] = to_dev(c)
+    assert buf[1:].data_ptr() % 16 == 8
+    torch.cuda.synchronize()
+    basis.gram(buf[1:].data_ptr(), basis.ngw, nst)
+    gpu_ctx.sync()
+    assert rel_err(from_dev(buf[1:].contiguous(), basis.ngw, nst), oh.gram(c, True)) <= 1e-11
+    basis.close()

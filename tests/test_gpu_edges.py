@@ -485,3 +485,45 @@ def test_spheres_just_past_half_the_edge(gpu_ctx, grid, ecut, nlx, real, nb):
         assert rel_err(rho.cpu().numpy(), rho_ref) <= tol
     ham.close()
     basis.close()
+
+
+@pytest.mark.parametrize("n,np2,ecut,nb,real", [
+    (24, 18, 12.0, 3, True), (28, 20, 25.0, 2, False), (30, 24, 25.0, 5, True),
+    (32, 18, 25.0, 4, False), (42, 20, 25.0, 7, True), (50, 28, 60.0, 3, False),
+    (54, 20, 25.0, 5, True), (56, 30, 60.0, 2, False), (66, 24, 25.0, 3, True),
+    (70, 20, 25.0, 4, False), (90, 18, 25.0, 5, True), (96, 30, 60.0, 2, False),
+    (100, 24, 25.0, 3, True)])
+def test_plane_every_edge(gpu_ctx, n, np2, ecut, nb, real):
+    """Local Hψ and density in the plane kernel at the edges the tests above leave out (each is
+    an instantiation with its own rows, padding and wavefronts)."""
+    import torch
+    from oracle import hpsi as oh
+    from oracle.basis import Basis as OB, FFTMaps, UnitCell
+    from qball_amd import Basis, Hamiltonian
+    from qball_amd.workload import make_system
+    sysm = make_system(ncell=1, ecut_ry=ecut, nbands=nb, seed=49, complex_basis=not real)
+    maps = FFTMaps(OB(UnitCell(sysm.a), sysm.ecut, force_complex=not real), n, n, np2)
+    r, c = sysm.rods, sysm.psi
+    basis = Basis(gpu_ctx, real, r["rod_h"], r["rod_k"], r["rod_lmin"], r["rod_size"],
+                  (n, n, np2), sysm.b)
+    v = np.random.default_rng(n).standard_normal(basis.N)
+    vd, cd = real_to_dev(v), to_dev(c)
+    hd = torch.zeros_like(cd)
+    rho = torch.zeros(basis.N, dtype=torch.float64, device="cuda")
+    ham = Hamiltonian(gpu_ctx, basis)
+    ham.set_vloc(vd.data_ptr())
+    torch.cuda.synchronize()
+    gpu_ctx.timing_report()
+    gpu_ctx.set_timing(True)
+    ham.hpsi(cd.data_ptr(), basis.ngw, nb, sysm.occ, hd.data_ptr(), basis.ngw, flags=0x4)
+    basis.density(cd.data_ptr(), basis.ngw, nb, sysm.occ, 1.0, sysm.omega, rho.data_ptr())
+    gpu_ctx.sync()
+    ran = gpu_ctx.timing_report()
+    gpu_ctx.set_timing(False)
+    assert {"plane_vmul", "plane_density"} <= set(ran)
+    ref = oh.rs_mul_add(maps, c, v, np.zeros_like(c))
+    assert rel_err(from_dev(hd, basis.ngw, nb), ref) <= 1e-12
+    assert rel_err(rho.cpu().numpy(),
+                   oh.compute_density(maps, c, sysm.occ, 1.0, sysm.omega)) <= 1e-12
+    ham.close()
+    basis.close()

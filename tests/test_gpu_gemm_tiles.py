@@ -76,3 +76,51 @@ def test_tiles(gpu_ctx, shape, real):
         assert np.linalg.norm(from_dev(hd, basis.ngw, nst) - 2 * ref) <= 2 * tol * size, flags
     ham.close()
     basis.close()
+
+
+# atoms, bands, cutoff; widths of the tiles of F and Hψ += βF in FP64, then in FP32
+WIDE = [(150, 200, 80.0, (128, 128), (128, 32)), (250, 390, 60.0, (128, 64), (128, 64)),
+        (200, 390, 60.0, (64, 64), (64, 64)), (100, 100, 60.0, (32, 64), (32, 32))]
+
+
+@pytest.mark.parametrize("natoms,nst,ecut,tiles64,tiles32", WIDE)
+def test_wide_tiles(gpu_ctx, natoms, nst, ecut, tiles64, tiles32):
+    """The 64 and 128 wide tiles of both products over several tiles and slices (Γ), with the
+    tiles that ran."""
+    import torch
+    from helpers import make_gpu_basis, product_tile
+    from qball_amd import Hamiltonian
+    from qball_amd.workload import make_system
+    lproj = [0, 1, 1, 1]
+    sysm = make_system(ncell=1, ecut_ry=ecut, nbands=nst, seed=33)
+    P, Q = 4 * natoms, 2 * sysm.ngw
+    for fp32, tiles in ((0, tiles64), (1, tiles32)):
+        assert (product_tile(fp32, P, nst, Q)[0], product_tile(2 + fp32, nst, Q, P)[0]) == tiles
+    rng = np.random.default_rng(34)
+    tau = rng.uniform(0.0, 10.0, (natoms, 3))
+    twnl = rng.standard_normal((4, sysm.ngw)) / (1.0 + sysm.g2)
+    wt = rng.uniform(-1.0, 1.0, 4)
+    ph = -(torch.from_numpy(sysm.kpg).cuda() @ torch.from_numpy(tau).cuda().T)
+    ph = torch.complex(torch.cos(ph), torch.sin(ph)).T
+    t = torch.from_numpy(twnl).cuda()
+    beta = torch.view_as_real(torch.cat([(-1j) ** l * t[i] * ph for i, l in enumerate(lproj)]))
+    psi = torch.view_as_real(torch.from_numpy(np.ascontiguousarray(sysm.psi.T)).cuda())
+    beta, psi = beta.reshape(P, Q), psi.reshape(nst, Q)
+    D = torch.from_numpy(np.repeat(wt, natoms) / sysm.omega).cuda()
+    F = 2.0 * beta @ psi.T - beta[:, :1] @ psi[:, :1].T
+    ref = ((D[:, None] * F).T @ beta).cpu().numpy().view(np.complex128).T
+    size = float(((D.abs()[:, None] * (2.0 * beta.abs() @ psi.abs().T)).T @ beta.abs()).norm())
+    basis = make_gpu_basis(gpu_ctx, sysm)
+    ham = Hamiltonian(gpu_ctx, basis)
+    ham.set_projectors([natoms], [4], lproj, wt, twnl.ravel(), tau.ravel(), sysm.omega)
+    ham.set_tuning("fnl_algo", 17)
+    ham.set_tuning("enl_algo", 17)
+    cd = to_dev(sysm.psi)
+    for flags, tol in ((0x1, 1e-15), (0x11, 5e-7)):
+        hd = torch.full_like(cd, np.nan)
+        torch.cuda.synchronize()
+        ham.hpsi(cd.data_ptr(), basis.ngw, nst, sysm.occ, hd.data_ptr(), basis.ngw, flags=flags)
+        gpu_ctx.sync()
+        assert np.linalg.norm(from_dev(hd, basis.ngw, nst) - ref) <= tol * size, flags
+    ham.close()
+    basis.close()

@@ -103,15 +103,6 @@ int main() {
     assert int(rc) != 0 and float(enl) != 42.0 and int(msg) > 0
 
 
-def product_tile(which, R, C, Q):
-    from qball_amd import lib
-    s = ctypes.c_int()
-    f = lib().qbh_product_tile
-    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long,
-                  ctypes.POINTER(ctypes.c_int)]
-    return f(which, R, C, Q, ctypes.byref(s)), s.value
-
-
 @pytest.mark.parametrize("which,R,C,Q,tile,slices", [
     # measured slower on 64-wide tiles: FP32 slices of 5500 to 9088 (F and the product after it),
     # FP64 with few workgroups a CU (4 slices 3.13 ms, large tile with 24 2.86)
@@ -125,6 +116,7 @@ def product_tile(which, R, C, Q):
 def test_product_tiles(which, R, C, Q, tile, slices):
     """Tile and slice rule of the matrix-core products at measured shapes (None: either tile,
     with at least that many slices)."""
+    from helpers import product_tile
     got = product_tile(which, R, C, Q)
     if tile is None:
         assert got[1] >= slices
