@@ -196,7 +196,8 @@ __device__ __forceinline__ void stage_b(cplx<T>* b, const cplx<T>* tw, int k1) {
 // a[k] *= W_n^{DIR e k}, k < K, n the length of the table tw (e (K - 1) < n).  FP64 and TAB read
 // every power from the table: local Hψ is 1.2 to 1.9 times closer to 64-bit reference transforms
 // than with the repeated products of w = tw[e] that FP32 forms otherwise (140^3: 5.3e-16 against
-// 8.2e-16 of the result), in the same time (140^3 x pass, 300 slots, 3.75 against 3.73 ms).
+// 8.2e-16 of the result), in the same time up to edge 180 (140^3 x pass, 300 slots, 3.75 against
+// 3.73 ms); from 192 on local Hψ takes 3 to 12 % longer (256^3, 32 bands 5.24 against 4.78 ms).
 template <int K, int DIR, bool TAB = false, typename T>
 __device__ __forceinline__ void twiddle_row(cplx<T>* a, const cplx<T>* tw, int e) {
   if (e == 0) return;

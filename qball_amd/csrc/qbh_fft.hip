@@ -178,8 +178,8 @@ static long plane_work(const GridDev& g, const PlaneOps* p) {
   return (long)g.np0 * g.nlx * p->wgs / 8;
 }
 
-// plane forms of the call `use` for nslots slots of this basis and precision, or null.  FP32 keeps
-// the passes: the plane's forward y transform has another radix order, which rounds differently.
+// plane forms of the call `use` for nslots slots of this basis and precision, or null (FP32 has
+// none).
 //
 // A plane is one chain of dependent stages in one workgroup; the passes take three launches instead
 // and spread the same work over more workgroups.  So the plane pays where its chain is short

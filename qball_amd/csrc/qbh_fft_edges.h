@@ -1,10 +1,11 @@
 // Grid edges with a two-factor register transform, n = N1*N2 with both factors from the
-// small DFTs of fft_reg.h (at most 16): every even length up to 180 that the reference's
-// factorisation rule accepts (2^k with at most 3^2, 5, 7 and 11, Basis.cc:126-154) except
-// 162, and the common longer ones; odd and other lengths take the LDS Stockham passes, which
-// make one LDS round trip per radix instead of three per transform pair: at 88^3 (108 Al
-// atoms, 195 bands, FP64, MI355X) the x pass took 1.37 ms and the y passes 0.30 / 0.26 ms per
-// Hψ on Stockham passes, and a two-cycle SCF 41.1 ms against 28.6 ms on the register ones.
+// small DFTs of fft_reg.h (at most 16): of the even lengths that the reference's factorisation
+// rule accepts (2^k with at most 3^2, 5, 7 and 11, Basis.cc:126-154) those from 18 to 256 except
+// 22, 198, 220 and 252, and of the longer products of 2, 3 and 5 also 50, 54, 100, 108 and 150.
+// All others take the LDS Stockham passes, which make one LDS round trip per radix instead of
+// three per transform pair: at 88^3 (108 Al atoms, 195 bands, FP64, MI355X) the x pass took 1.37
+// ms and the y passes 0.30 / 0.26 ms per Hψ on Stockham passes, and a two-cycle SCF 41.1 ms
+// against 28.6 ms on the register ones.
 // FP32 takes the same transforms at the E lengths.  At the D lengths (FP64 only) its factors are
 // those of F, whose transform keeps the radix order, tabled twiddles and so the rounding of the
 // Stockham passes that FP32 ran on there (stockham_order): its first factor is the product of

@@ -1051,10 +1051,10 @@ k_xload2(GridDev g, cplx<T>* __restrict__ t2, int nslots, int slots_per_wg,
 // ------------------------------------------------------------------------------------
 // x pass of band sums of products of transforms, without a grid per band:
 //   part[range][d][r] = sum_s w_s Re (IM: Im) (conj(a_s(r)) b_{d,s}(r)),  d < NB
-// over the slots with w_s > 0 of a range per blockIdx.y (w null: 1).  a and the b_d are y-transformed lines
-// (T2); a workgroup takes the NB + 1 fields of a slot one after the other through the same
-// row buffers, the next field's lines in flight, holds a(r) in registers and accumulates in
-// FP64.  Against storing the transforms as grids and multiplying them from memory (16 bytes a
+// over the slots with w_s > 0 of a range per blockIdx.y (w null: 1).  a and the b_d are
+// y-transformed lines (T2); a workgroup takes the NB + 1 fields of a slot one after the other
+// through the same row buffers, the next field's lines in flight, holds a(r) in registers and
+// accumulates in FP64.  Against storing the transforms as grids and multiplying them from memory (16 bytes a
 // point and band written and read, per field), MI355X: current
 // density of 128 bands at 72^3 2.90 -> 1.54 ms, of 64 bands at 60^3 1.19 -> 0.55; TD gradient of
 // 64 Si atoms, two steps, 103 -> 87 ms.  Bound like k_xpass2 by vector issue; at two waves per

@@ -122,8 +122,9 @@ int nl_lt_builtin_algo(Ctx* c) {
 // Built-in choice of both projector products: the matrix-core kernels of qbh_gemm.hip for
 // the real Γ view, rocBLAS for complex bases.
 int nl_builtin_algo(Ham* h, int which) {
-  // complex bases: rocBLAS for Hψ += βF, which ran 0.145 against 0.216 ms per call (Si64
-  // TD, beside the concurrent transforms) while F = βᴴψ ran 0.137 against 0.226 ms here
+  // complex bases: rocBLAS for Hψ += βF.  Alone this library's 64-wide tile is faster (0.115
+  // against 0.145 ms, 64 Si atoms), but beside the transforms it costs them more: ETRS steps 8.70
+  // against 8.58 ms, TD gradient 79.7 against 78.8.  F = βᴴψ ran 0.137 ms here against 0.226
   return (which == 1 && !h->b->g.real) ? 0 : kOwnGemm;
 }
 
